@@ -344,220 +344,160 @@ extern "C" int clarus_hip_boxmean(const void* x, int32_t x_dtype, void* out, int
   return check_launch("boxmean");
 }
 
-// Sliding-window variant for dilation 1 and narrow rows. A lane owns 8
-// consecutive channels of ONE input half (with a gate, lanes l and l + 32 hold the two halves of
-// the same output channels) and walks a run of R consecutive pixels along a row: per step it
-// loads one new column of 3 pixels (3 16-byte loads per output instead of 9 per half) and adds
-// it to the up to 3 outputs whose window contains that column, so 3 partial outputs are live.
-// Its 72 tap weights and 8 biases stay in registers for the whole run. SimpleGate / GELU gate
-// combine the halves with a cross-lane exchange (l <-> l ^ 32). The 8 lanes of a pixel read
-// 128 contiguous bytes per half; a wave covers 8 (gate: 4) runs of 64 channels.
-// Per output the taps are summed column by column (kx outer, ky inner) after the bias.
-template <int XDT, int GATE, int R>
-__global__ void __launch_bounds__(256) dw_rows_kernel(const DwP p) {
-  constexpr int XES = (XDT == DT_BF16) ? 2 : 4;
-  constexpr int RPW = GATE ? 4 : 8;  // runs per wave
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int hf = GATE ? (lane >> 5) : 0;
-  const int l = GATE ? (lane & 31) : lane;
-  const int cg = l & 7, rw = l >> 3;
-  const int cout = (int)p.cout, cin = (int)p.cin;
-  const int nslices = (cout + DW_SLICE - 1) / DW_SLICE;
-  const int slice = blockIdx.x % nslices;
-  const int c0 = slice * DW_SLICE + cg * 8;      // first output channel of the lane
-  const bool active = c0 < cout;                 // the same for both halves of a pair
-  const int ci = c0 + (GATE ? hf * cout : 0);    // first input channel of the lane's half
-  float wt[9][8], bs[8];
-#pragma unroll
-  for (int t = 0; t < 9; ++t)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) wt[t][i] = active ? p.w[(int64_t)t * cin + ci + i] : 0.f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) bs[i] = (active && p.b) ? p.b[ci + i] : 0.f;
-
-  const int H = (int)p.h, W = (int)p.w_;
-  const int rpr = (W + R - 1) / R;               // runs per image row
-  const int total = (int)p.n * H * rpr;          // the host checks that this fits 31 bits
-  const int per_wg = 4 * RPW;
-  const int stride = (gridDim.x / nslices) * per_wg;
-  const unsigned char* X = (const unsigned char*)p.x;
-  for (int run = (blockIdx.x / nslices) * per_wg + wave * RPW + rw; run < total; run += stride) {
-    const int img = run / (H * rpr);
-    const int rr = run - img * H * rpr;
-    const int y = rr / rpr;
-    const int x0 = (rr - y * rpr) * R;
-    const unsigned char* rowp[3];
-    bool rok[3];
-#pragma unroll
-    for (int ky = 0; ky < 3; ++ky) {
-      const int yy = y + ky - 1;
-      rok[ky] = active && yy >= 0 && yy < H;
-      rowp[ky] = X + ((int64_t)(img * H + (rok[ky] ? yy : 0)) * W * cin + ci) * XES;
-    }
-    // every load of the run is issued before the first FMA (one memory round trip per run)
-    RawFrag<XDT> raw[R + 2][3];
-#pragma unroll
-    for (int cc = 0; cc < R + 2; ++cc) {
-      const int x = x0 - 1 + cc;
-      const bool xok = x >= 0 && x < W;
-#pragma unroll
-      for (int ky = 0; ky < 3; ++ky)
-        raw[cc][ky] = (xok && rok[ky]) ? raw_load<XDT>(rowp[ky] + (int64_t)x * cin * XES) : raw_zero<XDT>();
-    }
-    float acc[3][8];
-#pragma unroll
-    for (int cc = 0; cc < R + 2; ++cc) {  // column x0 - 1 + cc
-      if (cc < R) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[cc % 3][i] = bs[i];
-      }
-      f32x8 col[3];
-#pragma unroll
-      for (int ky = 0; ky < 3; ++ky) col[ky] = raw_f32<XDT>(raw[cc][ky]);
-#pragma unroll
-      for (int j = cc - 2; j <= cc; ++j) {  // outputs whose window holds this column (kx = cc - j)
-        if (j < 0 || j >= R) continue;
-#pragma unroll
-        for (int ky = 0; ky < 3; ++ky)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) acc[j % 3][i] = fmaf(wt[ky * 3 + cc - j][i], col[ky].v[i], acc[j % 3][i]);
-      }
-      if (cc < 2) continue;
-      // output j = cc - 2 is complete
-      const int j = cc - 2;
-      float v[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = acc[j % 3][i];
-      if constexpr (GATE != 0) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float o = __shfl_xor(v[i], 32, 64);  // the other half of the same channel
-          v[i] = GATE == 1 ? v[i] * o : gelu_erf(v[i]) * o;
-        }
-      } else if (p.act == ACT_GELU) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = gelu_erf(v[i]);
-      }
-      const int xo = x0 + j;
-      if (hf != 0 || !active || xo >= W) continue;
-      const int64_t oo = ((int64_t)(img * H + y) * W + xo) * cout + c0;
-      if (p.o_dt == DT_BF16) {
-        u32x4 q;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          q[i] = (unsigned)f32_to_bf16_bits(v[2 * i]) | ((unsigned)f32_to_bf16_bits(v[2 * i + 1]) << 16);
-        *reinterpret_cast<u32x4*>((unsigned short*)p.out + oo) = q;
-      } else {
-        float* op = (float*)p.out + oo;
-        *reinterpret_cast<f32x4*>(op) = f32x4{v[0], v[1], v[2], v[3]};
-        *reinterpret_cast<f32x4*>(op + 4) = f32x4{v[4], v[5], v[6], v[7]};
-      }
-    }
-  }
-}
-
-// LDS-tiled variant for bf16 input with a gate. A workgroup owns a slice of 64 output channels
-// and walks tiles of TH x DWT_TW output pixels. The tile's input (its rows and columns plus a
-// one-pixel halo, both input halves: (TH + 2) x (DWT_TW + 2) pixels x 256 bytes) is copied
-// global -> LDS once by direct copies, pixels outside the image from a zero page, so every input
-// vector crosses the vector-memory path once per tile instead of 9 times. With NBUF = 2 the next
-// tile's copies go out before the current tile is computed. Lane (run, cq) owns output column
-// `run` of the tile and channels 4 cq .. 4 cq + 3 of both halves, keeps their 72 taps and 8
-// biases in registers and walks its column down the tile: per input row six 8-byte LDS reads
-// (both halves of the pixels left, at and right of the column; the next row's issued before this
-// row's FMAs) feed the up to 3 outputs whose window holds that row, and the gate is formed in the
-// lane. In LDS a pixel's two 128-byte halves are swapped when its column is odd, so the 4 runs of
-// a wave read both bank halves. Per output the sum runs bias, then ky outer, kx inner (the order of
-// dwconv3x3_kernel). Stores are buffer stores whose range drops the lanes outside the image, so
-// every wave issues the same TH stores per tile and the wait for the next tile's copies can leave
+// LDS-tiled form for dilation 1. A workgroup owns a slice of channels and walks tiles of TH x tw output
+// pixels. A lane owns one output column of the tile and 8 input channels (with a gate 4 of each half,
+// and the gate is formed in the lane; without one 8 consecutive), so cq lanes serve a column's slice of
+// 8 cq input channels and tw = 256 / cq columns fit a workgroup; cq is chosen per channel count so that
+// few lanes idle (144 channels: 18 lanes x 14 columns, not 2 x 64 of 128). The lane keeps its 72 taps and
+// 8 biases in registers and walks its column down the tile: per input row the pixels left, at and right
+// of the column come from LDS (the next row's reads issued before this row's FMAs) and feed the up to 3
+// outputs whose window holds that row. Per output the sum runs bias, then ky outer, kx inner (the order
+// of dwconv3x3_kernel).
+// Copies. The tile's input with a one-pixel halo ((TH + 2) x (tw + 2) pixels) is copied global -> LDS
+// once by direct 16-byte copies, pixels outside the image from a zero page; with NBUF = 2 the next tile's
+// copies go out before the current tile is computed. With a gate a pixel's two halves are swapped in LDS
+// when its column is odd, so neighbouring columns read both bank halves.
+// Stores are buffer stores whose range ends at the tile's last image row and which drop lanes outside the
+// image, so every wave issues the same stores per tile and the wait for the next tile's copies can leave
 // them in flight.
-constexpr int DWT_TW = 16;
-template <int TH>
+// XCD-aware dealing: workgroup L runs on XCD L mod 8, which gets a contiguous eighth of the tiles (all
+// slices), so the halo rows and columns that neighbouring tiles share, and the 128-byte lines that
+// neighbouring slices share, are read into one L2 mostly once. A multiple of 8 slices is dealt by slice
+// instead, XCD = slice mod 8: the same sharing of halos, and the eighths stay in step whatever the tile
+// count (a whole NAFNet block at 90 x 160, 512 channels: 150.6 us against 153.9 by eighths). Eighths against
+// 64 consecutive tiles per XCD and round (the GPU sweeping top to bottom): Restormer's block 983 / 998 us.
+// Bound: HBM for bf16 without a gate or with SimpleGate (C in and out, 2C in and C out); with the GELU gate
+// VALU work comes near it (18 FMAs, 6 bf16 unpacks and ~25 slots of GELU per output). Measured (us, 720 x
+// 1280 bf16, before -> now): 288 channels no gate 547 (one thread per pixel and 8 channels) -> 251, 4.2 TB/s;
+// 144 no gate 254 (register windows along rows) -> 114, 4.6 TB/s; SimpleGate 128 -> 64 90 -> 81, 4.4 TB/s
+// (tiles dealt round-robin over the XCDs before); GELU gate 256 -> 128 280 -> 206; fp32 144 491 -> 211.
+template <int XDT, int TH>
 struct DwTile {
-  static constexpr int ROWS = TH + 2, COLS = DWT_TW + 2;
-  static constexpr int UNITS = ROWS * COLS * 2 * 8;    // 16-byte units: pixel, half, 8 units of 128 B
-  static constexpr int COPIES = (UNITS + 255) / 256;   // copies per lane (4 waves of 64 units each)
+  static constexpr int ROWS = TH + 2;
+  static constexpr int UL = XDT == DT_BF16 ? 1 : 2;               // 16-byte units per lane and pixel
+  static constexpr int COPIES = ((ROWS * 288 + 255) / 256) * UL;  // copies per lane: (tw + 2) cq <= 288
   static constexpr int BYTES = COPIES * 256 * 16;
 };
 static __device__ __attribute__((aligned(256))) unsigned char g_dw_zero[256];
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));  // taps and bias need no alignment
 
-template <int GATE, int TH, int NBUF, int ODT>
-__global__ void __launch_bounds__(256) dw_tile_kernel(const DwP p) {
-  static_assert(GATE == 1 || GATE == 2, "gated form only");
-  using G = DwTile<TH>;
-  constexpr int OES = ODT == DT_BF16 ? 2 : 4;
+struct DwTileP {
+  int cq, tw, nslices, streams;            // lanes per column, columns, slices, tile streams per dealing unit
+  int xw;                                  // dealing units: 8 XCDs, or 1 (dealt by slice)
+  int tiles_y, tiles_x, ptiles;
+  unsigned mag_u, mag_c;                   // ceil(2^19 / (units per pixel)), ceil(2^19 / (tw + 2))
+};
+
+template <int XDT, int GATE, int TH, int NBUF, int ODT>
+__global__ void __launch_bounds__(256, 2) dw_tile_kernel(const DwP p, const DwTileP g) {
+  using G = DwTile<XDT, TH>;
+  constexpr int XES = XDT == DT_BF16 ? 2 : 4, OES = ODT == DT_BF16 ? 2 : 4;
+  constexpr int SPR = (GATE == 0 && ODT == DT_F32) ? 2 : 1;  // stores per output row of a lane
+  constexpr int EU = 16 / XES;                                // channels per 16-byte unit
   __shared__ __attribute__((aligned(16))) unsigned char tile[NBUF][G::BYTES];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int cq = lane & 15, run = wave * 4 + (lane >> 4);
+  const int col = (int)threadIdx.x / g.cq, l = (int)threadIdx.x - col * g.cq;
   const int cout = (int)p.cout, cin = (int)p.cin;
-  const int nslices = (cout + DW_SLICE - 1) / DW_SLICE;
-  const int slice = blockIdx.x % nslices;
-  const int c0 = slice * DW_SLICE + cq * 4;  // first output channel of the lane
-  const bool active = c0 < cout;             // cout % 8 == 0: all 4 channels or none
-  float wt[2][9][4], bs[2][4];               // [half][tap][channel]
+  const int sc = (GATE ? 4 : 8) * g.cq;          // output channels of a slice
+  const int xcd = blockIdx.x & (g.xw - 1), local = blockIdx.x / g.xw;
+  const int slice = local % g.nslices;
+  const int cs = slice * sc;
+  const int c0 = cs + l * (GATE ? 4 : 8);        // first output channel of the lane
+  const bool active = c0 < cout && col < g.tw;   // cout % 8 == 0: all of the lane's channels or none
+  float wt[2][9][4], bs[2][4];                   // [half][tap][channel]; lanes past cout hold its last ones
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int ci = c0 + h * cout;
+    const int ci = min(c0, cout - (GATE ? 4 : 8)) + h * (GATE ? cout : 4);
 #pragma unroll
     for (int t = 0; t < 9; ++t) {
-      const f32x4 a = active ? *reinterpret_cast<const f32x4*>(p.w + (int64_t)t * cin + ci) : f32x4{0.f, 0.f, 0.f, 0.f};
+      const f32x4_u a = *reinterpret_cast<const f32x4_u*>(p.w + (int64_t)t * cin + ci);
 #pragma unroll
       for (int i = 0; i < 4; ++i) wt[h][t][i] = a[i];
     }
-    const f32x4 b = (active && p.b) ? *reinterpret_cast<const f32x4*>(p.b + ci) : f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4_u b = {0.f, 0.f, 0.f, 0.f};
+    if (p.b) b = *reinterpret_cast<const f32x4_u*>(p.b + ci);
 #pragma unroll
     for (int i = 0; i < 4; ++i) bs[h][i] = b[i];
   }
-
   const int H = (int)p.h, W = (int)p.w_;
-  const int tiles_x = (W + DWT_TW - 1) / DWT_TW, tiles_y = (H + TH - 1) / TH;
-  const int ptiles = (int)p.n * tiles_y * tiles_x;  // the host checks that this fits 31 bits
-  const int stride = gridDim.x / nslices;
   const unsigned char* X = (const unsigned char*)p.x;
-  // the host checks that the output is under 2^31 - 16 bytes: 32-bit buffer offsets
-  const __amdgpu_buffer_rsrc_t orc = buf_rsrc_n(p.out, (uint32_t)(p.n * p.h * p.w_ * p.cout * OES));
-  // copy j of a lane fills unit u = (wave + 4 j) * 64 + lane of the tile's LDS image: pixel u / 16
-  // of the (TH + 2) x (DWT_TW + 2) halo tile, 16 bytes (u % 8) of half ((u / 8) % 2) ^ (column % 2)
-  // of the slice's 128
-  const int k = lane & 7, slot = (lane >> 3) & 1;
-  const bool k_real = slice * DW_SLICE + k * 8 < cout;
+  const int upp = g.cq * G::UL, colw = g.tw + 2;   // 16-byte units per pixel, halo columns
   auto tile_pos = [&](int t, int& img, int& y0, int& x0) __attribute__((always_inline)) {
-    img = t / (tiles_y * tiles_x);
-    const int rem = t - img * tiles_y * tiles_x;
-    const int ty = rem / tiles_x;
+    img = t / (g.tiles_y * g.tiles_x);
+    const int rem = t - img * g.tiles_y * g.tiles_x;
+    const int ty = rem / g.tiles_x;
     y0 = ty * TH;
-    x0 = (rem - ty * tiles_x) * DWT_TW;
+    x0 = (rem - ty * g.tiles_x) * g.tw;
   };
+  // copy j of a lane fills unit u = (wave + 4 j) * 64 + lane of the LDS image: pixel u / upp of the halo
+  // tile and unit u % upp of its channels (with a gate unit k of slot 0 / 1 is half (k's slot) ^ (column % 2))
+  // off: byte offset of each copy from the halo tile's first pixel; rc: its row << 8 | column. Units that hold
+  // no pixel or channel: offset 0, column 255
+  unsigned off[G::COPIES], rc[G::COPIES];
+#pragma unroll
+  for (int j = 0; j < G::COPIES; ++j) {
+    const unsigned u = (unsigned)((wave + 4 * j) * 64 + lane);
+    const int pix = (int)(__umul24(u, g.mag_u) >> 19), k = (int)u - __mul24(pix, upp);
+    const int r = (int)(__umul24((unsigned)pix, g.mag_c) >> 19), c = pix - __mul24(r, colw);
+    int kk = k, seg = 0;
+    if constexpr (GATE != 0) {
+      const int hu = upp >> 1, slot = k >= hu ? 1 : 0;
+      kk = k - slot * hu;
+      seg = slot ^ (c & 1);
+    }
+    const int cc = cs + kk * EU;
+    const bool real = cc < cout && r < G::ROWS;
+    off[j] = real ? (unsigned)(((r * W + c) * cin + cc + seg * cout) * XES) : 0u;
+    rc[j] = real ? (unsigned)(r << 8 | c) : 255u;
+  }
   auto issue = [&](int t, unsigned char* dst) __attribute__((always_inline)) {
     int img, y0, x0;
     tile_pos(t, img, y0, x0);
+    const unsigned char* base = X + ((((int64_t)img * H + y0 - 1) * W + x0 - 1) * cin) * XES;
+    const bool inside = y0 >= 1 && y0 + TH < H && x0 >= 1 && x0 + g.tw < W;  // the whole halo tile is
 #pragma unroll
     for (int j = 0; j < G::COPIES; ++j) {
-      const int pix = ((wave + 4 * j) * 64 + lane) >> 4;
-      const int r = pix / G::COLS, c = pix - (pix / G::COLS) * G::COLS;
-      const int seg = slot ^ (c & 1);
-      const int yy = y0 - 1 + r, xx = x0 - 1 + c;
-      const bool ok = k_real && pix < G::ROWS * G::COLS && yy >= 0 && yy < H && xx >= 0 && xx < W;
-      const int yc = min(max(yy, 0), H - 1), xc = min(max(xx, 0), W - 1);  // an address in the image
-      const unsigned char* src =
-          ok ? X + (((int64_t)img * H + yc) * W + xc) * cin * 2 + (slice * DW_SLICE + seg * cout + k * 8) * 2 : g_dw_zero;
+      const unsigned char* src = base + off[j];
+      if (!inside) {
+        const int c = (int)(rc[j] & 255u), yy = y0 - 1 + (int)(rc[j] >> 8), xx = x0 - 1 + c;
+        if (c == 255 || (unsigned)yy >= (unsigned)H || (unsigned)xx >= (unsigned)W) src = g_dw_zero;
+      }
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                        (__attribute__((address_space(3))) void*)(dst + (wave + 4 * j) * 1024), 16, 0, 0);
     }
   };
-  // byte offset of half h of tile pixel (row, column) for this lane's channels
-  auto lds_at = [&](int row, int col, int h) __attribute__((always_inline)) {
-    return (row * G::COLS + col) * 256 + ((h ^ (col & 1)) * 128) + cq * 8;
+  const int lcol = min(col, g.tw - 1);            // lanes past the last column read the last one
+  const int rpitch = colw * upp * 16;
+  typedef typename std::conditional<XDT == DT_BF16, u32x2, u32x4>::type Raw4;  // 4 channels as loaded
+  auto load_row = [&](const unsigned char* cur, int row, Raw4 (&q)[3][2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx) {
+      const unsigned char* px = cur + row * rpitch + (lcol + dx) * upp * 16;
+      if constexpr (GATE != 0) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          q[dx][h] = *reinterpret_cast<const Raw4*>(px + ((h ^ ((lcol + dx) & 1)) * (upp >> 1)) * 16 + l * 4 * XES);
+      } else if constexpr (XDT == DT_BF16) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(px + l * 16);
+        q[dx][0] = Raw4{v[0], v[1]};
+        q[dx][1] = Raw4{v[2], v[3]};
+      } else {
+        q[dx][0] = *reinterpret_cast<const Raw4*>(px + l * 32);
+        q[dx][1] = *reinterpret_cast<const Raw4*>(px + l * 32 + 16);
+      }
+    }
   };
-  int t = blockIdx.x / nslices;
-  if (NBUF == 2 && t < ptiles) issue(t, tile[0]);
-  for (int it = 0; t < ptiles; ++it, t += stride) {
+  // this dealing unit's tiles [lo, hi), every `streams`-th of them this workgroup's
+  const int lo = (int)((int64_t)g.ptiles * xcd / g.xw), hi = (int)((int64_t)g.ptiles * (xcd + 1) / g.xw);
+  int t = lo + local / g.nslices;
+  if (NBUF == 2 && t < hi) issue(t, tile[0]);
+  for (int it = 0; t < hi; ++it, t += g.streams) {
     unsigned char* cur = tile[NBUF == 2 ? (it & 1) : 0];
     if constexpr (NBUF == 2) {
-      // this tile's copies are older than the previous tile's TH stores
-      if (it == 0) wait_vmcnt<0>(); else wait_vmcnt<TH>();
+      // this tile's copies are older than the previous tile's stores
+      if (it == 0) wait_vmcnt<0>(); else wait_vmcnt<TH * SPR>();
       __syncthreads();  // copies landed; every wave is done with the other buffer
-      if (t + stride < ptiles) issue(t + stride, tile[(it & 1) ^ 1]);
+      if (t + g.streams < hi) issue(t + g.streams, tile[(it & 1) ^ 1]);
     } else {
       issue(t, cur);
       wait_vmcnt<0>();
@@ -565,23 +505,21 @@ __global__ void __launch_bounds__(256) dw_tile_kernel(const DwP p) {
     }
     int img, y0, x0;
     tile_pos(t, img, y0, x0);
-    const int xo = x0 + run;
+    const int xo = x0 + col;
+    // output rows y0 .. of this image, TH of them or up to its last (the host checks the range's size)
+    const int64_t orow = (int64_t)W * cout * OES;
+    const __amdgpu_buffer_rsrc_t orc = buf_rsrc_n((unsigned char*)p.out + ((int64_t)img * H + y0) * orow,
+                                                  (uint32_t)(min(TH, H - y0) * orow));
+    const int ocol = (active && xo < W) ? (xo * cout + c0) * OES : 0x7ffffff0;
     float acc[3][2][4];
-    u32x2 q[2][3][2];  // [row parity][dx][half]: raw bf16 of the row being summed and the next
-#pragma unroll
-    for (int dx = 0; dx < 3; ++dx)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) q[0][dx][h] = *reinterpret_cast<const u32x2*>(cur + lds_at(0, run + dx, h));
-#pragma unroll
-    for (int ir = 0; ir < G::ROWS; ++ir) {  // input row y0 - 1 + ir
-      if (ir + 1 < G::ROWS) {
-#pragma unroll
-        for (int dx = 0; dx < 3; ++dx)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            q[(ir + 1) & 1][dx][h] = *reinterpret_cast<const u32x2*>(cur + lds_at(ir + 1, run + dx, h));
-      }
-      if (ir < TH) {
+    // [row parity][dx][half]: bf16: the row being summed and the next; fp32: the row (registers)
+    constexpr int AHEAD = XDT == DT_BF16 ? 1 : 0;
+    Raw4 q[1 + AHEAD][3][2];
+    if constexpr (AHEAD != 0) load_row(cur, 0, q[0]);
+    static_for<G::ROWS>([&](auto IR) __attribute__((always_inline)) {  // input row y0 - 1 + ir
+      constexpr int ir = IR.value;
+      if constexpr (ir + AHEAD < G::ROWS) load_row(cur, ir + AHEAD, q[(ir + 1) & AHEAD]);
+      if constexpr (ir < TH) {
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -592,49 +530,96 @@ __global__ void __launch_bounds__(256) dw_tile_kernel(const DwP p) {
       for (int dx = 0; dx < 3; ++dx)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const u32x2 r = q[ir & 1][dx][h];
-          v[dx][h][0] = __uint_as_float(r[0] << 16);
-          v[dx][h][1] = __uint_as_float(r[0] & 0xffff0000u);
-          v[dx][h][2] = __uint_as_float(r[1] << 16);
-          v[dx][h][3] = __uint_as_float(r[1] & 0xffff0000u);
+          const Raw4 r = q[ir & AHEAD][dx][h];
+          if constexpr (XDT == DT_BF16) {
+            v[dx][h][0] = __uint_as_float(r[0] << 16);
+            v[dx][h][1] = __uint_as_float(r[0] & 0xffff0000u);
+            v[dx][h][2] = __uint_as_float(r[1] << 16);
+            v[dx][h][3] = __uint_as_float(r[1] & 0xffff0000u);
+          } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[dx][h][i] = __uint_as_float(r[i]);
+          }
         }
+      static_for<3>([&](auto KY) __attribute__((always_inline)) {  // outputs whose window holds this row
+        constexpr int ky = 2 - KY.value, o = ir - ky;
+        if constexpr (o >= 0 && o < TH) {
 #pragma unroll
-      for (int o = ir - 2; o <= ir; ++o) {  // outputs whose window holds this row (ky = ir - o)
-        if (o < 0 || o >= TH) continue;
+          for (int dx = 0; dx < 3; ++dx)
 #pragma unroll
-        for (int dx = 0; dx < 3; ++dx)
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-          for (int h = 0; h < 2; ++h)
+              for (int i = 0; i < 4; ++i)
+                acc[o % 3][h][i] = fmaf(wt[h][ky * 3 + dx][i], v[dx][h][i], acc[o % 3][h][i]);
+        }
+      });
+      if constexpr (ir >= 2) {
+        constexpr int o = ir - 2;  // output row y0 + o is complete
+        const int oo = ocol == 0x7ffffff0 ? ocol : ocol + o * (int)orow;
+        float(&a)[2][4] = acc[o % 3];
+        if constexpr (GATE != 0) {
+          float r[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              acc[o % 3][h][i] = fmaf(wt[h][(ir - o) * 3 + dx][i], v[dx][h][i], acc[o % 3][h][i]);
+          for (int i = 0; i < 4; ++i) r[i] = GATE == 1 ? a[0][i] * a[1][i] : gelu_erf(a[0][i]) * a[1][i];
+          if constexpr (ODT == DT_BF16)
+            __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack2_bf16(r[0], r[1]), pack2_bf16(r[2], r[3])}, orc, oo, 0, 0);
+          else
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, f32x4{r[0], r[1], r[2], r[3]}), orc, oo, 0, 0);
+        } else {
+          if (p.act == ACT_GELU) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) a[h][i] = gelu_erf(a[h][i]);
+          }
+          if constexpr (ODT == DT_BF16) {
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4{pack2_bf16(a[0][0], a[0][1]), pack2_bf16(a[0][2], a[0][3]),
+                                                         pack2_bf16(a[1][0], a[1][1]), pack2_bf16(a[1][2], a[1][3])},
+                                                   orc, oo, 0, 0);
+          } else {
+            __builtin_amdgcn_raw_buffer_store_b128(
+                __builtin_bit_cast(u32x4, f32x4{a[0][0], a[0][1], a[0][2], a[0][3]}), orc, oo, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(
+                __builtin_bit_cast(u32x4, f32x4{a[1][0], a[1][1], a[1][2], a[1][3]}), orc, oo, 16, 0);
+          }
+        }
       }
-      if (ir < 2) continue;
-      const int o = ir - 2;  // output row y0 + o is complete
-      float g[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float a = acc[o % 3][0][i], b = acc[o % 3][1][i];
-        if constexpr (GATE == 1) g[i] = a * b;
-        else g[i] = gelu_erf(a) * b;
-      }
-      const int yo = y0 + o;
-      const bool keep = active && yo < H && xo < W;
-      const int oo = keep ? (int)(((((int64_t)img * H + yo) * W + xo) * cout + c0) * OES) : 0x7ffffff0;
-      if constexpr (ODT == DT_BF16) {
-        u32x2 w2;
-        w2[0] = (unsigned)f32_to_bf16_bits(g[0]) | ((unsigned)f32_to_bf16_bits(g[1]) << 16);
-        w2[1] = (unsigned)f32_to_bf16_bits(g[2]) | ((unsigned)f32_to_bf16_bits(g[3]) << 16);
-        __builtin_amdgcn_raw_buffer_store_b64(w2, orc, oo, 0, 0);
-      } else {
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, f32x4{g[0], g[1], g[2], g[3]}), orc, oo, 0, 0);
-      }
-    }
+    });
     if constexpr (NBUF == 1) __syncthreads();  // every wave is done with the tile before the next copies land
   }
 }
 
-constexpr int DW_RUN = 4;  // pixels per run of dw_rows_kernel
+// Lanes per column, columns and slices of dw_tile_kernel for `units` lane units of channels (4 output
+// channels with a gate, else 8), and its tile height, returned. A workgroup takes as long for a tile
+// whatever lanes idle: the cost counts tiles (at least the 512 workgroups that run at once) times a tile's
+// rows. cq is even with a gate (16-byte copies of halves) and at least 16 where the channels reach it:
+// 256 bytes of a pixel or more per slice (us, 720p bf16 without a gate, 9 lanes -> 18: 288 channels
+// 296 -> 250, 144 channels 131 -> 114). Heights: bf16 6 rows, or 2 where 6 leave CUs without a tile
+// (32 x 42, 512 channels, gate: 8.7 -> 6.9 us); fp32, whose 6-row tile fills half a CU's LDS, 2 rows
+// (90 x 160: 1152 channels 35.2 -> 30.0, 2048 with a GELU gate 69.0 -> 51.5).
+static int dw_tile_shape(int64_t units, int64_t n, int64_t H, int64_t W, bool gate, bool f32, DwTileP& g) {
+  double best = 1e300;
+  int th = 2;
+  const int lo = (int)std::min<int64_t>(gate ? units + (units & 1) : units, 16);
+  for (int cq = std::max(lo, 2); cq <= 26; ++cq) {
+    const int tw = 256 / cq;
+    if ((gate && cq % 2) || (tw + 2) * cq > 288) continue;
+    const int64_t nsl = cdiv(units, cq);
+    for (int t = 2; t <= (f32 ? 2 : 6); t += 4) {
+      const double tiles = (double)nsl * (double)(n * cdiv(H, t) * cdiv(W, tw));
+      if (t == 2 && !f32 && nsl * n * cdiv(H, 6) * cdiv(W, tw) >= 256) continue;
+      const double cost = std::max(tiles / 512.0, 1.0) * (t + 3.0) * (1.0 + 0.5 / tw);
+      if (cost < best * 0.999) {
+        best = cost;
+        th = t;
+        g.cq = cq;
+        g.tw = tw;
+        g.nslices = (int)nsl;
+      }
+    }
+  }
+  return th;
+}
 
 extern "C" int clarus_hip_dwconv3x3(const void* x, int32_t x_dtype, const float* w, const float* bias, void* out,
                                     int32_t o_dtype, int64_t n, int64_t h, int64_t wd, int64_t c, int32_t dil,
@@ -672,24 +657,26 @@ extern "C" int clarus_hip_dwconv3x3(const void* x, int32_t x_dtype, const float*
     const unsigned blocks = (unsigned)(nslices * std::min<int64_t>(chunks, cap));                               \
     hipLaunchKernelGGL(fn, dim3(blocks), dim3(256), 0, s, p);                                                   \
   } while (0)
-  // sliding-window kernel for dilation 1 and up to 256 input channels (measured on the NAFNet
-  // 720p levels: 127 vs 151 us at 128 channels, even at 256, slower from 512 channels on, where
-  // the per-pixel kernel's higher occupancy wins): runs of DW_RUN pixels, workgroups of 16
-  // (gate) / 32 runs
-  // LDS-tiled kernel: bf16 input with a gate, dilation 1, 16-byte aligned taps and bias, an
-  // output under 2^31 - 16 bytes (32-bit buffer offsets). Tiles of 6 rows, two buffers (two
-  // workgroups per CU at 225 VGPRs; NAFNet-w64 720p levels 0-4, cold, us: 91 / 50 / 31 / 19 / 14
-  // against 128 / 73 / 45 / 28 / 17 for the kernels below; 8-row tiles with one buffer 95 / 51 /
-  // 32 / 20 / 13)
-  const int64_t o_bytes = n * h * wd * cout * (o_dtype == DT_BF16 ? 2 : 4);
-  if (dil == 1 && gate != 0 && x_dtype == DT_BF16 && aligned(w, 16) && (!bias || aligned(bias, 16)) &&
-      o_bytes < ((int64_t)1 << 31) - 16) {
-    constexpr int TH = 6, NBUF = 2;
-    const int64_t ptiles = n * cdiv(h, TH) * cdiv(wd, DWT_TW);
-    CLARUS_REQUIRE(ptiles < ((int64_t)1 << 31), "dwconv3x3: problem too large for 32-bit tile indexing");
-#define DW_TILE(G, ODT)                                                                                         \
+  // LDS-tiled kernel: every call with dilation 1 whose tile rows fit 2^31-byte buffer ranges and whose
+  // tile count fits 30 bits (it needs no alignment of taps and bias); the per-pixel kernel keeps dilated
+  // taps, whose halo would be larger than the tile, and images past those ranges. Down to 24 x 30 pixels
+  // the tiled form is the faster or even (us, before -> now: fp32 144 channels 10.6 -> 7.2, 288 channels at
+  // 24 x 49 6.9 -> 7.3, bf16 7.1 -> 6.7).
+  {
+    const int oes = o_dtype == DT_BF16 ? 2 : 4;
+    DwTileP g{};
+    const int th = dw_tile_shape(cdiv(cout, gate ? 4 : 8), n, h, wd, gate != 0, x_dtype == DT_F32, g);
+    const int64_t ptiles = n * cdiv(h, th) * cdiv(wd, g.tw);
+    if (dil == 1 && (th + 2) * (wd + 2) * c * 4 < ((int64_t)1 << 31) && ptiles < ((int64_t)1 << 30)) {
+      g.tiles_y = (int)cdiv(h, th);
+      g.tiles_x = (int)cdiv(wd, g.tw);
+      g.ptiles = (int)ptiles;
+      const unsigned upp = (unsigned)g.cq * (x_dtype == DT_BF16 ? 1 : 2);
+      g.mag_u = ((1u << 19) + upp - 1) / upp;
+      g.mag_c = ((1u << 19) + (unsigned)g.tw + 1) / ((unsigned)g.tw + 2);
+#define DW_TILE(XDT, G, TH, NBUF, ODT)                                                                          \
   do {                                                                                                          \
-    auto fn = &dw_tile_kernel<G, TH, NBUF, ODT>;                                                                \
+    auto fn = &dw_tile_kernel<XDT, G, TH, NBUF, ODT>;                                                           \
     static const int per_cu = [&] {                                                                             \
       int k = 0;                                                                                                \
       if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, reinterpret_cast<const void*>(fn), 256, 0) !=       \
@@ -698,45 +685,29 @@ extern "C" int clarus_hip_dwconv3x3(const void* x, int32_t x_dtype, const float*
         k = 1;                                                                                                  \
       return k;                                                                                                 \
     }();                                                                                                        \
-    const int64_t cap = std::max<int64_t>(1, (int64_t)device_cus() * per_cu / nslices);                        \
-    const unsigned blocks = (unsigned)(nslices * std::min<int64_t>(ptiles, cap));                               \
-    hipLaunchKernelGGL(fn, dim3(blocks), dim3(256), 0, s, p);                                                   \
+    g.xw = g.nslices % 8 ? 8 : 1;                                                                               \
+    const int64_t cap = std::max<int64_t>(1, (int64_t)device_cus() * per_cu / (g.xw * g.nslices));             \
+    g.streams = (int)std::min<int64_t>(cdiv(ptiles, g.xw), cap);                                                \
+    hipLaunchKernelGGL(fn, dim3((unsigned)(g.xw * g.nslices * g.streams)), dim3(256), 0, s, p, g);              \
   } while (0)
-    note_kernel("dw_tile_kernel gate=%d th=%d nbuf=%d", gate, TH, NBUF);
-    if (o_dtype == DT_BF16) {
-      if (gate == 1) DW_TILE(1, DT_BF16); else DW_TILE(2, DT_BF16);
-    } else {
-      if (gate == 1) DW_TILE(1, DT_F32); else DW_TILE(2, DT_F32);
-    }
+#define DW_TILE_G(XDT, TH, NBUF, ODT)                                                                           \
+  do {                                                                                                          \
+    if (gate == 0) DW_TILE(XDT, 0, TH, NBUF, ODT);                                                              \
+    else if (gate == 1) DW_TILE(XDT, 1, TH, NBUF, ODT);                                                         \
+    else DW_TILE(XDT, 2, TH, NBUF, ODT);                                                                        \
+  } while (0)
+      note_kernel("dw_tile_kernel gate=%d th=%d cq=%d tw=%d", gate, th, g.cq, g.tw);
+      if (x_dtype == DT_BF16 && th == 6) {
+        if (o_dtype == DT_BF16) DW_TILE_G(DT_BF16, 6, 2, DT_BF16); else DW_TILE_G(DT_BF16, 6, 2, DT_F32);
+      } else if (x_dtype == DT_BF16) {
+        if (o_dtype == DT_BF16) DW_TILE_G(DT_BF16, 2, 2, DT_BF16); else DW_TILE_G(DT_BF16, 2, 2, DT_F32);
+      } else {
+        if (o_dtype == DT_BF16) DW_TILE_G(DT_F32, 2, 1, DT_BF16); else DW_TILE_G(DT_F32, 2, 1, DT_F32);
+      }
+#undef DW_TILE_G
 #undef DW_TILE
-    return check_launch("dwconv3x3");
-  }
-  if (dil == 1 && c <= 256) {
-    const int64_t runs = n * h * cdiv(wd, DW_RUN);
-    CLARUS_REQUIRE(runs < ((int64_t)1 << 31), "dwconv3x3: problem too large for 32-bit run indexing");
-    const int64_t rchunks = cdiv(runs, gate ? 16 : 32);
-#define DW_ROWS(XDT, G)                                                                                         \
-  do {                                                                                                          \
-    auto fn = &dw_rows_kernel<XDT, G, DW_RUN>;                                                                  \
-    static const int per_cu = [&] {                                                                             \
-      int k = 0;                                                                                                \
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, reinterpret_cast<const void*>(fn), 256, 0) !=       \
-              hipSuccess ||                                                                                     \
-          k < 1)                                                                                                \
-        k = 1;                                                                                                  \
-      return k;                                                                                                 \
-    }();                                                                                                        \
-    const int64_t cap = std::max<int64_t>(1, (int64_t)device_cus() * per_cu / nslices);                                        \
-    const unsigned blocks = (unsigned)(nslices * std::min<int64_t>(rchunks, cap));                              \
-    hipLaunchKernelGGL(fn, dim3(blocks), dim3(256), 0, s, p);                                                   \
-  } while (0)
-    if (x_dtype == DT_BF16) {
-      if (gate == 1) DW_ROWS(DT_BF16, 1); else if (gate == 2) DW_ROWS(DT_BF16, 2); else DW_ROWS(DT_BF16, 0);
-    } else {
-      if (gate == 1) DW_ROWS(DT_F32, 1); else if (gate == 2) DW_ROWS(DT_F32, 2); else DW_ROWS(DT_F32, 0);
+      return check_launch("dwconv3x3");
     }
-#undef DW_ROWS
-    return check_launch("dwconv3x3");
   }
   if (x_dtype == DT_BF16) {
     if (gate == 1) DW_LAUNCH(DT_BF16, 1); else if (gate == 2) DW_LAUNCH(DT_BF16, 2); else DW_LAUNCH(DT_BF16, 0);

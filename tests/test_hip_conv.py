@@ -205,9 +205,8 @@ def test_config5_upconv(h, w, hip_bf16):
                                           (False, "gelu", 1), (False, None, 2)])
 def test_dwconv(dt, gate, act, dil, c, hip_bf16, hip_f32):
     """Depthwise 3x3 + SimpleGate / GELU gate / GELU / dilation 2 (tools/test_kernels.py:110-121,
-    193-199), odd sizes (two images of 37 x 53, partial tiles at both edges): bf16 with a gate
-    takes the LDS-tiled kernel; otherwise 96 channels take the sliding-window kernel (dilation
-    1), 528 and 640 the per-pixel one."""
+    193-199), odd sizes (two images of 37 x 53, partial tiles at both edges): with a gate and
+    without one dilation 1 takes the LDS-tiled kernel, dilation 2 the per-pixel one."""
     hip = hip_bf16 if dt == torch.bfloat16 else hip_f32
     g = gen(8)
     x, w, b = rnd(g, 2, 37, 53, c, dtype=dt), rnd(g, c, 1, 3, 3), rnd(g, c)
@@ -254,6 +253,28 @@ def test_dwconv_tile_edges(n, h, w, c, gate, hip_bf16):
     got = hip_bf16.dwconv(x.cuda(), wt.cuda(), None if b is None else b.cuda(), gate=gate)
     assert _lib.last_kernel().startswith("dw_tile_kernel"), _lib.last_kernel()
     check(got.cpu(), TorchRef(torch.float32, "cpu").dwconv(x, wt, b, gate=gate), f"dwconv {n}x{h}x{w}x{c} gate={gate}")
+
+
+@pytest.mark.parametrize("n,h,w,c,gate,act", [
+    (1, 1, 1, 8, False, None), (1, 3, 2, 16, False, "gelu"),         # smallest slices, images inside one tile
+    (2, 13, 15, 144, False, None), (1, 7, 29, 288, False, None),     # 18 lanes x 14 columns, remainders
+    (1, 26, 33, 1152, False, None), (1, 12, 40, 216, False, "gelu"),  # several slices, the last one partial
+    (1, 5, 40, 32, "gelu", None), (2, 9, 17, 528, "gelu", None), (1, 40, 70, 512, True, None)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_dwconv_tile_forms(n, h, w, c, gate, act, dt, hip_bf16, hip_f32):
+    """dw_tile_kernel without a gate, with fp32 rows and at both tile heights, at the edges of its tiles and
+    channel slices, the bias at an address that is 4-byte aligned only."""
+    from clarus_amd import _lib
+    g = gen(c + h)
+    x = rnd(g, n, h, w, c, dtype=dt)
+    wt, b = rnd(g, c, 1, 3, 3, scale=0.3), rnd(g, c, scale=0.5)
+    off = torch.zeros(c + 1)
+    off[1:] = b
+    hip = hip_bf16 if dt == torch.bfloat16 else hip_f32
+    got = hip.dwconv(x.cuda(), wt.cuda(), off.cuda()[1:], gate=gate, act=act)
+    assert _lib.last_kernel().startswith("dw_tile_kernel"), _lib.last_kernel()
+    check(got.cpu(), TorchRef(torch.float32, "cpu").dwconv(x, wt, b, gate=gate, act=act),
+          f"dwconv tile {n}x{h}x{w}x{c} gate={gate} act={act} {dt}")
 
 
 def test_dwconv_bf16_in_fp32_out(hip_bf16):
