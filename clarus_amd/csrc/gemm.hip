@@ -7,6 +7,7 @@
 #include "gemm_lds_dispatch.hpp"
 #include "gemm_stream_dispatch.hpp"
 #include "gemm_rowstream_dispatch.hpp"
+#include "gemm_rowwide_dispatch.hpp"
 
 namespace clarus {
 
@@ -261,6 +262,20 @@ extern "C" int clarus_hip_gemm(const ClarusGemmArgs* a, void* stream) {
     if (a->tile == 18 || (a->tile == 0 && slice_shape && a->m <= 80000)) {
       note_kernel("gemm_slice_kernel k=%lld c=%s", (long long)a->k, a->c_dtype == DT_BF16 ? "bf16" : "f32");
       CLARUS_REQUIRE(launch_gemm_slice(p, (hipStream_t)stream), "gemm: W-slice launch");
+      return check_launch("gemm");
+    }
+  }
+  // all-channel row kernel (tile 19 forces it): 16 < K <= 96 with bf16 weights and no gate, without a
+  // prologue, with LN / RMS, or the LN-multiply of fp32 rows. Automatic without a residual, with the
+  // LN-multiply, and with a residual up to K = 48 (us, 720 x 1280, ring streaming kernel / this one: 48 -> 48
+  // 53.0 / 50.5, 32 -> 32 46 / 34; at K = 64 71.1 / 72.4, which keeps the ring)
+  {
+    const bool wide_ok = a->a_mode == CLARUS_A_ROWS && a->batch == 1 && !a->gate && !pro_round &&
+                         gemm_rowwide_fits(p, a->a_dtype, a->w_dtype);
+    CLARUS_REQUIRE(a->tile != 19 || wide_ok, "gemm: the all-channel row kernel does not take this problem");
+    const bool wide_auto = a->tile == 0 && wide_ok && (!a->res || a->k <= 48 || a->pro == PRO_LNMUL);
+    if (a->tile == 19 || wide_auto) {
+      CLARUS_REQUIRE(launch_gemm_rowwide(p, a->a_dtype, (hipStream_t)stream), "gemm: all-channel row kernel launch");
       return check_launch("gemm");
     }
   }

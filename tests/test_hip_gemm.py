@@ -1699,3 +1699,53 @@ def test_config2_nafnet_gemms(c, h, w, hip_bf16):
     print(f"[config2] c{c}: expand -> {kernels[0]}; c->c -> {kernels[1]}")
     if c == 512:
         assert kernels[1].startswith("wstream_kernel gate=0 res=0"), kernels[1]
+
+
+# ------------------------------------------------------------------ all-channel row kernel (16 < K <= 96)
+@pytest.mark.parametrize("m,k,n,opts", [
+    (1, 24, 8, {}), (31, 40, 24, {"ln": True}), (33, 96, 576, {"ln": True}), (129, 88, 104, {"ln": "rms"}),
+    (700, 48, 144, {"ln": True}), (65, 64, 200, {"act": "gelu"}), (97, 32, 32, {"res": "bf16", "scale": True}),
+    (200, 48, 56, {"res": "fp32", "out": "fp32", "scale": True}), (130, 96, 264, {"out": "fp32"}),
+    (33000, 48, 72, {"ln": True}), (32771, 64, 168, {}),   # tiles stored as one run of memory
+    (33000, 48, 128, {"ln": True})])
+def test_rowwide_kernel(m, k, n, opts, hip_bf16):
+    """linear on gemm_rowwide_kernel: remainders of its 32-pixel tiles, 32-channel tiles, 16-k steps and
+    channel chunks, every epilogue, against the oracle in fp32 on the same bf16 operands. Products are
+    fp32-accurate (hi + lo rows), so a result is one rounding of the oracle's value."""
+    from clarus_amd import _lib
+    g = torch.Generator().manual_seed(m + k + n)
+    x = torch.randn(1, 1, m, k, generator=g).bfloat16()
+    w = (torch.randn(k, n, generator=g) / k ** 0.5).bfloat16()
+    b = torch.randn(n, generator=g) * 0.1
+    sc = torch.randn(n, generator=g) * 0.5 if opts.get("scale") else None
+    dts = {"bf16": torch.bfloat16, "fp32": torch.float32}
+    res = torch.randn(1, 1, m, n, generator=g).to(dts[opts["res"]]) if "res" in opts else None
+    odt = dts[opts.get("out", "bf16")]
+    dev = lambda t: None if t is None else t.cuda()  # noqa: E731
+    got = hip_bf16.linear(x.cuda(), w.cuda(), b.cuda(), ln=opts.get("ln", False), act=opts.get("act"), scale=dev(sc),
+                          residual=dev(res), out_dtype=odt)
+    assert _lib.last_kernel().startswith("gemm_rowwide_kernel"), _lib.last_kernel()
+    ref = TorchRef(torch.float32, "cpu").linear(x, w, b, ln=opts.get("ln", False), act=opts.get("act"), scale=sc,
+                                                residual=res, out_dtype=torch.float32)
+    if odt == torch.float32:
+        assert_fp32(got.cpu(), ref, what=f"rowwide {m}x{k}x{n} {opts}")
+    else:
+        assert_bf16(got.cpu(), ref, f"rowwide {m}x{k}x{n} {opts}")
+
+
+@pytest.mark.parametrize("m,k,n,act", [(1, 24, 8, None), (95, 96, 48, None), (130, 72, 40, "gelu")])
+def test_rowwide_ln_mul(m, k, n, act, hip_bf16):
+    """ln_mul_linear of fp32 rows by a channel slice of a wider bf16 tensor on gemm_rowwide_kernel."""
+    from clarus_amd import _lib
+    g = torch.Generator().manual_seed(m + k)
+    x = torch.randn(1, 1, m, k, generator=g) * 100
+    wide = torch.randn(1, 1, m, 3 * k, generator=g).bfloat16()
+    lw, lb = 1 + 0.1 * torch.randn(k, generator=g), 0.1 * torch.randn(k, generator=g)
+    w = (torch.randn(k, n, generator=g) / k ** 0.5).bfloat16()
+    res = torch.randn(1, 1, m, n, generator=g).bfloat16()
+    got = hip_bf16.ln_mul_linear(x.cuda(), lw.cuda(), lb.cuda(), wide.cuda()[..., 2 * k:], w.cuda(), m_act=act,
+                                 residual=res.cuda())
+    assert _lib.last_kernel().startswith("gemm_rowwide_kernel pro=5"), _lib.last_kernel()
+    ref = TorchRef(torch.float32, "cpu").ln_mul_linear(x, lw, lb, wide[..., 2 * k:], w, m_act=act, residual=res,
+                                                       out_dtype=torch.float32)
+    assert_bf16(got.cpu(), ref, f"rowwide ln_mul {m}x{k}x{n}")
