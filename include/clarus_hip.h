@@ -357,8 +357,9 @@ int clarus_hip_patch_filter(const void* x, int32_t x_dtype, int64_t ldx, const f
  * (h, w >= 9), which for a per-pixel GEMM is the GEMM of the reflected pixels. out [batch, h, w, n]
  * contiguous (o_dtype); residual contiguous like out or NULL. k % 8 == 0. With bf16 weights the
  * GEMM's A values enter bf16 MFMAs as hi + lo pairs where they are not bf16 already (2^-16
- * relative per operand); with fp32 weights it runs on fp32 MFMAs. The DFT products are those of
- * clarus_hip_patch_filter.
+ * relative per operand); with fp32 weights it runs on fp32 MFMAs. With bf16 x and weights and k <= 96
+ * (192 without a prologue) the transforms run as fp32 FFTs, which need the gains only (fwd and inv being
+ * the matrices of rfft2 and irfft2); otherwise as the DFT products of clarus_hip_patch_filter.
  * replaces kernels/freq.py:189-273 ln_gemm_patch_filter (ops/triton_cuda.py:260-272)
  */
 int clarus_hip_linear_patch_filter(const void* x, int32_t x_dtype, const void* wt, int32_t w_dtype,

@@ -337,3 +337,23 @@ def test_patch_corr(dt, hip_bf16, hip_f32):
     for name, fn in [("batch stride 2HWC", lambda t: t[::2]), ("batch stride 0", lambda t: t[:1].expand(3, -1, -1, -1)),
                      ("channel slice", lambda t: t[..., 8:8 + 2 * c]), ("H/W transposed", lambda t: t.transpose(1, 2))]:
         assert_fp32(hip.patch_corr(fn(bd), c).cpu(), REF.patch_corr(fn(base), c), rel=1e-5, what=f"patch_corr {name}")
+
+
+@pytest.mark.parametrize("h,w,k,n,ln,res", [
+    (9, 9, 8, 8, False, False), (17, 40, 24, 40, True, False), (45, 61, 48, 288, True, True),
+    (24, 40, 96, 72, "rms", False), (33, 16, 192, 40, False, True), (200, 192, 48, 33, True, False),
+    (168, 200, 88, 40, True, False), (176, 184, 136, 24, False, False), (168, 200, 16, 8, "rms", True)])
+def test_fft_lpf_kernel(h, w, k, n, ln, res, hip_bf16):
+    """linear_patch_filter with FFT patch transforms: one patch per workgroup and several (over 512 patches),
+    partial batches, channel tiles and 16-k steps, reflected edges, against the oracle in fp32 on the same bf16
+    operands (gains without the symmetry of a real filter's spectrum in columns 0 and 4)."""
+    from clarus_amd import _lib
+    g = gen(h + k + n)
+    x, f = rnd(g, 1, h, w, k).bfloat16(), rnd(g, n, 8, 5)
+    wl, b = rnd(g, k, n, scale=k ** -0.5).bfloat16(), rnd(g, n, scale=0.1)
+    rr = rnd(g, 1, h, w, n).bfloat16() if res else None
+    got = hip_bf16.linear_patch_filter(x.cuda(), wl.cuda(), b.cuda(), f.cuda(), ln=ln, ln_eps=1e-5,
+                                       residual=None if rr is None else rr.cuda())
+    assert _lib.last_kernel().startswith("fft_lpf_kernel"), _lib.last_kernel()
+    ref = REF.linear_patch_filter(x, wl, b, f, ln=ln, ln_eps=1e-5, residual=rr)
+    assert_bf16(got.cpu(), ref, f"fft lpf {h}x{w} k{k} n{n}")
