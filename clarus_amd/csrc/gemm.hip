@@ -8,6 +8,7 @@
 #include "gemm_stream_dispatch.hpp"
 #include "gemm_rowstream_dispatch.hpp"
 #include "gemm_rowwide_dispatch.hpp"
+#include "gemm_smallm_dispatch.hpp"
 
 namespace clarus {
 
@@ -278,6 +279,12 @@ extern "C" int clarus_hip_gemm(const ClarusGemmArgs* a, void* stream) {
       CLARUS_REQUIRE(launch_gemm_rowwide(p, a->a_dtype, (hipStream_t)stream), "gemm: all-channel row kernel launch");
       return check_launch("gemm");
     }
+  }
+  if (a->tile == 20) {  // few rows of K = 128 / 256 (by request only: its prologue output is rounded once to bf16)
+    CLARUS_REQUIRE(a->a_mode == CLARUS_A_ROWS && a->batch == 1 && gemm_smallm_fits(p, a->a_dtype, a->w_dtype),
+                   "gemm: the few-row kernel does not take this problem");
+    launch_gemm_smallm(p, a->a_dtype, a->gate != 0, (hipStream_t)stream);
+    return check_launch("gemm");
   }
   int tile_override = 0;
   if (a->tile == 0 && plain_bf16 && a->res && a->k <= 128 && (!run_div || run_div % 16 == 0)) tile_override = 3;

@@ -123,6 +123,12 @@ class HipOps(Backend):
     # without its round trip through HBM); False keeps the separate pass (K = 128) or the 128-pixel
     # kernel's prologue (K = 256). NAFNet-w64 levels 1 and 2, conv1 and conv4.
     wres_prologue = True
+    # Few rows of K = 128 / 256 with bf16 weights on gemm_smallm_kernel, the LayerNorm, RMS or bf16 map prologue
+    # of bf16 or fp32 rows inside it (rounded once to bf16, as the separate pass writes it): the deep levels of
+    # small images, where the persistent kernels and the pass before them are a chain of latencies. Up to one
+    # workgroup (128 rows x 32 channels) per CU (us, other kernels / this one, LayerNorm of fp32 rows 256 -> 512:
+    # 1344 rows 10.5 / 8.2, 3072 rows 11.2 / 15.1; 128 -> 256: 3072 rows 7.7 / 5.6, 6144 rows 8.2 / 8.2).
+    smallm = True
     # linear_patch_filter as one kernel (GEMM output straight into the patch DFT); False runs
     # linear (fp32 output) and patch_filter as two ops.
     fuse_patch_filter = True
@@ -274,6 +280,20 @@ class HipOps(Backend):
             return None
         return "wr", self._wr_pack(w, bool(gate))
 
+    def _small_m(self, x, w, pro, sm, k, nout, gate, act, m, res) -> bool:
+        """This linear goes to gemm_smallm_kernel (see smallm). Plain square GEMMs without residual, gate or
+        activation (the NAFNet SCA GEMMs) stay on the W-slice kernel."""
+        if not (self.smallm and k in (128, 256) and w.dtype == torch.bfloat16 and nout % 8 == 0
+                and not self.prologue_split and self.split_min_k <= k and (res is None or _vec16(res))):
+            return False
+        if -(-m // 128) * -(-nout // 32) > self._cu_count():
+            return False
+        if pro in (_lib.PRO_LN, _lib.PRO_RMS):
+            return True
+        if x.dtype != torch.bfloat16 or (pro == _lib.PRO_MUL and sm.dtype != torch.bfloat16):
+            return False
+        return pro == _lib.PRO_MUL or res is not None or gate or act != 0 or nout != k
+
     def _wp_mul(self, x, w, pro, sm, k, nout, gate, act, m, res):
         """("wp" | "wr", W^T packed) when this map-prologue linear runs with the multiply inside the
         kernel its separate pass would feed (see wstream_mul, wres_mul), else None."""
@@ -296,11 +316,14 @@ class HipOps(Backend):
                 and x.dtype in (torch.bfloat16, torch.float32) and w.dtype == torch.bfloat16
                 and act in (0, _lib.ACT_GELU)):
             return None
-        if self._cus is None:
-            self._cus = torch.cuda.get_device_properties(self.dev).multi_processor_count
-        if 4 * -(-m // 128) * (nw // 512) < 3 * self._cus:
+        if 4 * -(-m // 128) * (nw // 512) < 3 * self._cu_count():
             return None
         return "wp", self._w2p(w, bool(gate))
+
+    def _cu_count(self) -> int:
+        if self._cus is None:
+            self._cus = torch.cuda.get_device_properties(self.dev).multi_processor_count
+        return self._cus
 
     # ------------------------------------------------------------------ GEMMs
     def _linear_plan(self, x, w, bias, ln, act, gate, scale, residual, mul, out_dtype):
@@ -364,6 +387,9 @@ class HipOps(Backend):
         epi = dict(bias=self._bias(bias), scale=self._bias(scale), res=residual, ldr=nout, gate=gate,
                    act=_lib.ACT_GELU if act == "gelu" else 0)
         m = n * h * wd
+        if self._small_m(x, w, pro, sm, k, nout, gate, epi["act"], m, residual):
+            return self._gemm("linear", a=x, wt=self._wt(w), c=out, m=m, n=nout, k=k, lda=k, ldc=nout, pro=pro, small=sm,
+                              geom=geom, ln_eps=float(ln_eps), tile=20, **epi)
         if self._prologue_pass(w, pro, k):
             wpp = (self._wr_prologue(x, w, pro, k, nout, gate, epi["act"], residual)
                    or self._wp_prologue(x, w, pro, k, nout, gate, epi["act"], m, residual)

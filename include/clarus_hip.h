@@ -110,7 +110,10 @@ typedef struct ClarusGemmArgs {
                          14 / 15 the same with 256 / 128 pixels x 256 channels per tile,
                          16 / 17 streaming with a per-wave LDS ring (K <= 128 bf16 / 64 fp32;
                          17: 4 channel blocks per workgroup), 18 W-slice (bf16 A and W, no
-                         prologue / gate / act / residual, K = 128 / 256 / 512, N % 64 == 0) */
+                         prologue / gate / act / residual, K = 128 / 256 / 512, N % 64 == 0),
+                         19 all channels per 32 rows (16 < K <= 96, bf16 W, no gate), 20 few rows
+                         (K = 128 / 256, bf16 W; no prologue, LN, RMS or a bf16 map, its output
+                         rounded once to bf16 as clarus_hip_rows_prologue's rows) */
 } ClarusGemmArgs;
 
 /* replaces kernels/gemm.py:353-400 fused_gemm and :403-429 _gemm_wide */

@@ -1749,3 +1749,44 @@ def test_rowwide_ln_mul(m, k, n, act, hip_bf16):
     ref = TorchRef(torch.float32, "cpu").ln_mul_linear(x, lw, lb, wide[..., 2 * k:], w, m_act=act, residual=res,
                                                        out_dtype=torch.float32)
     assert_bf16(got.cpu(), ref, f"rowwide ln_mul {m}x{k}x{n}")
+
+
+# ------------------------------------------------------------------ few-row kernel (K = 128 / 256)
+@pytest.mark.parametrize("m,k,n,kind,xdt", [
+    (1, 256, 512, "ln", "fp32"), (131, 128, 40, "ln", "bf16"), (300, 256, 264, "rms", "fp32"), (97, 256, 256, "lngate", "fp32"),
+    (640, 128, 72, "lngate", "bf16"), (129, 256, 256, "res32", "bf16"), (33, 128, 200, "res16", "bf16"),
+    (96, 256, 256, "mul", "bf16"), (96, 128, 24, "mul", "bf16"), (260, 256, 48, "gelu", "bf16")])
+def test_smallm_kernel(m, k, n, kind, xdt, hip_bf16):
+    """linear on gemm_smallm_kernel against the oracle on the rows its prologue rounds once to bf16: remainders
+    of its 128-row and 32-channel tiles, the gate, residuals of both types, the map multiply of two images."""
+    from clarus_amd import _lib
+    g = torch.Generator().manual_seed(m + k + n)
+    h, wd = (8, 6) if kind == "mul" else (1, m)
+    nb = m // (h * wd)
+    x = torch.randn(nb, h, wd, k, generator=g).to(torch.float32 if xdt == "fp32" else torch.bfloat16)
+    gate = kind == "lngate"
+    w = (torch.randn(k, 2 * n if gate else n, generator=g) / k ** 0.5).bfloat16()
+    b = torch.randn(w.shape[1], generator=g) * 0.1
+    sc = torch.randn(n, generator=g) * 0.3 if kind in ("res32", "mul") else None
+    res = None
+    if kind in ("res32", "res16", "mul"):
+        res = torch.randn(nb, h, wd, n, generator=g).to(torch.bfloat16 if kind == "res16" else torch.float32)
+    ln = {"ln": True, "lngate": True, "rms": "rms"}.get(kind, False)
+    ref_x, mul, dmul = x.float(), None, None
+    if kind == "mul":
+        mul = Small(torch.randn(nb, 4, 3, k, generator=g).bfloat16(), 2, 1, h, wd)
+        dmul = Small(mul.data.cuda(), 2, 1, h, wd)
+        ref_x = (ref_x * TorchRef.expand(mul).float()).bfloat16().float()
+    elif ln:
+        ref_x = TorchRef.ln(ref_x, 1e-6, rms=(ln == "rms")).bfloat16().float()
+    dev = lambda t: None if t is None else t.cuda()  # noqa: E731
+    got = hip_bf16.linear(x.cuda(), w.cuda(), b.cuda(), ln=ln, gate=gate, act="gelu" if kind == "gelu" else None,
+                          scale=dev(sc), residual=dev(res), mul=dmul, out_dtype=torch.float32)
+    assert _lib.last_kernel().startswith("gemm_smallm_kernel"), _lib.last_kernel()
+    ref = TorchRef(torch.float32, "cpu").linear(ref_x, w, b, gate=gate, act="gelu" if kind == "gelu" else None, scale=sc,
+                                                residual=res, out_dtype=torch.float32)
+    # an element of a LayerNorm row may round to the neighbouring bf16 value where the statistics' summation order
+    # differs: one step (2^-8 relative) of a few of its K terms; 2e-3 of the output scale bounds four of them
+    tol = 2e-3 if ln else 1e-5
+    e = ((got.cpu() - ref).abs().max() / ref.abs().max()).item()
+    assert e <= tol, f"smallm {m}x{k}x{n} {kind}: {e:.2e}"
