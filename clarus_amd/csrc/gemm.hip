@@ -4,6 +4,7 @@
 
 #include "capi.hpp"
 #include "gemm_dispatch.hpp"
+#include "gemm_f32_dispatch.hpp"
 #include "gemm_lds_dispatch.hpp"
 #include "gemm_stream_dispatch.hpp"
 #include "gemm_rowstream_dispatch.hpp"
@@ -367,6 +368,17 @@ extern "C" int clarus_hip_gemm(const ClarusGemmArgs* a, void* stream) {
     launch_row_stats(a->a, a->a_dtype, a->lda, a->m, a->k, a->pro == PRO_RMS, a->ln_eps, a->stats,
                      (hipStream_t)stream);
     p.stats = a->stats;
+  }
+  // fp32 operands with K > 128: the LDS-tiled fp32 kernel (tile 21 forces it) from 128 tiles of 64 pixels x 128
+  // channels on; with fewer the 64 x 64 tiles below fill more of the GPU (us, general / LDS-tiled: 3000 rows
+  // 384 -> 384, 141 tiles 31.0 / 24.8; 1176 rows 192 -> 576, 95 tiles 18.0 / 21.2; 384 -> 384, 57 tiles 21.2 / 23.4)
+  {
+    const bool f32_ok = a->a_mode == CLARUS_A_ROWS && !a->gate && gemm_f32_fits(p, a->a_dtype, a->w_dtype, a->batch);
+    CLARUS_REQUIRE(a->tile != 21 || f32_ok, "gemm: the LDS-tiled fp32 kernel does not take this problem");
+    if (a->tile == 21 || (a->tile == 0 && f32_ok && cdiv(a->m, 64) * cdiv(a->n, 128) * a->batch >= 128)) {
+      launch_gemm_f32(p, a->batch, (hipStream_t)stream);
+      return check_launch("gemm");
+    }
   }
   // bf16 operands without prologue: the DMA-pipelined kernels. K % 64 == 0 runs on 32x32x16
   // MFMAs with 64-k chunks (tile 13 forces it), other K % 32 == 0 on 16x16x32 MFMAs with 32-k

@@ -113,7 +113,8 @@ typedef struct ClarusGemmArgs {
                          prologue / gate / act / residual, K = 128 / 256 / 512, N % 64 == 0),
                          19 all channels per 32 rows (16 < K <= 96, bf16 W, no gate), 20 few rows
                          (K = 128 / 256, bf16 W; no prologue, LN, RMS or a bf16 map, its output
-                         rounded once to bf16 as clarus_hip_rows_prologue's rows) */
+                         rounded once to bf16 as clarus_hip_rows_prologue's rows), 21 LDS-tiled
+                         fp32 (fp32 A and W, K > 128, no gate; none, LN or RMS with stats) */
 } ClarusGemmArgs;
 
 /* replaces kernels/gemm.py:353-400 fused_gemm and :403-429 _gemm_wide */

@@ -1790,3 +1790,34 @@ def test_smallm_kernel(m, k, n, kind, xdt, hip_bf16):
     tol = 2e-3 if ln else 1e-5
     e = ((got.cpu() - ref).abs().max() / ref.abs().max()).item()
     assert e <= tol, f"smallm {m}x{k}x{n} {kind}: {e:.2e}"
+
+
+# ------------------------------------------------------------------ LDS-tiled fp32 kernel (K > 128)
+@pytest.mark.parametrize("m,k,n,kind", [
+    (8200, 136, 40, "plain"), (4100, 200, 136, "ln"), (2049, 384, 520, "rms"), (8193, 160, 128, "res"), (3000, 264, 392, "gelu"),
+    (16500, 136, 1160, "plain")])
+def test_gemm_f32_kernel(m, k, n, kind, hip_f32):
+    """linear in fp32 on gemm_f32_kernel (both tile heights): remainders of its pixel and channel tiles and of its
+    32-k chunks, statistics of the separate pass, residual and scale, GELU, against the oracle within 1e-5."""
+    from clarus_amd import _lib
+    g = torch.Generator().manual_seed(m + k)
+    x, w = torch.randn(1, 1, m, k, generator=g), torch.randn(k, n, generator=g) / k ** 0.5
+    b = torch.randn(n, generator=g) * 0.1
+    res = torch.randn(1, 1, m, n, generator=g) if kind == "res" else None
+    sc = torch.randn(n, generator=g) * 0.3 if kind == "res" else None
+    kw = dict(ln={"ln": True, "rms": "rms"}.get(kind, False), act="gelu" if kind == "gelu" else None)
+    dev = lambda t: None if t is None else t.cuda()  # noqa: E731
+    got = hip_f32.linear(x.cuda(), w.cuda(), b.cuda(), scale=dev(sc), residual=dev(res), **kw)
+    assert _lib.last_kernel().startswith("gemm_f32_kernel"), _lib.last_kernel()
+    assert_fp32(got.cpu(), TorchRef(torch.float32, "cpu").linear(x, w, b, scale=sc, residual=res, **kw), what=f"f32 {m}x{k}x{n} {kind}")
+
+
+def test_gemm_f32_per_image(hip_f32):
+    """linear_per_image in fp32 on gemm_f32_kernel: two images, a channel slice of a wider tensor, a residual."""
+    from clarus_amd import _lib
+    g = torch.Generator().manual_seed(3)
+    qkv = torch.randn(2, 50, 70, 3 * 144, generator=g)
+    w, res = torch.randn(2, 144, 144, generator=g) / 12, torch.randn(2, 50, 70, 144, generator=g)
+    got = hip_f32.linear_per_image(qkv.cuda()[..., 288:], w.cuda(), residual=res.cuda())
+    assert _lib.last_kernel().startswith("gemm_f32_kernel"), _lib.last_kernel()
+    assert_fp32(got.cpu(), TorchRef(torch.float32, "cpu").linear_per_image(qkv[..., 288:], w, residual=res), what="f32 per image")
