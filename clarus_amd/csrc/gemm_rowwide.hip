@@ -37,6 +37,7 @@ struct RwP {
 };
 
 constexpr int RW_W_MAX = 60 * 1024;
+constexpr int RW_LDS_MAX = 160 * 1024;  // of a CU
 constexpr int RW_ST_ROW = 128 + 16;  // bytes per pixel of a wave's store tile (not linear)
 
 template <int PRO, int TA, int KS, bool LIN>
@@ -295,16 +296,22 @@ __global__ void __launch_bounds__(256, LIN ? 2 : TA == DT_F32 ? 3 : KS <= 4 ? 4 
   }
 }
 
+// dynamic LDS of a workgroup: W^T, vectors, the four waves' store tiles
+template <int KS, bool LIN>
+int rw_lds(int ntc, int n) {
+  return ntc * KS * 1024 + (64 * ntc + 32 * KS) * 4 + 4 * 32 * (LIN ? n * 2 : RW_ST_ROW);
+}
+
 template <int PRO, int TA, int KS, bool LIN>
 void launch_rw(RwP& p, hipStream_t s) {
   auto fn = &gemm_rowwide_kernel<PRO, TA, KS, LIN>;
   static const bool set = [&] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, RW_LDS_MAX);
     return true;
   }();
   (void)set;
   const GemmP& g = p.g;
-  const int lds = p.ntc * KS * 1024 + (64 * p.ntc + 32 * KS) * 4 + 4 * 32 * (LIN ? (int)g.n * 2 : RW_ST_ROW);
+  const int lds = rw_lds<KS, LIN>(p.ntc, (int)g.n);
   int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(fn), 256, lds) != hipSuccess ||
       per_cu < 1)
@@ -326,9 +333,9 @@ void choose_rw(const GemmP& g, hipStream_t s) {
     // rows whose length is no multiple of 128 bytes: stored tile by tile as one run, so that no 128-byte line
     // is written in two parts (us, 720 x 1280, K = 48: N = 288 174 -> 142, N = 144 93 -> 85); the tile's store
     // buffer takes LDS, which costs more than it gives at K = 96 (360 x 640, N = 288: 48 -> 61) and where the
-    // row groups alone leave CUs idle
-    if (nt <= most && g.c_dt == DT_BF16 && g.ldc == g.n && g.n % 64 != 0 && g.n > 64 && !g.has_res && g.act == ACT_NONE &&
-        !g.scale && g.out_scale == 1.0f && cdiv(g.m, 128) >= 256) {
+    // row groups alone leave CUs idle. The store tiles of four waves have to fit LDS beside W^T (K = 48: N < 456)
+    if (nt <= most && rw_lds<KS, true>(nt, (int)g.n) <= RW_LDS_MAX && g.c_dt == DT_BF16 && g.ldc == g.n &&
+        g.n % 64 != 0 && g.n > 64 && !g.has_res && g.act == ACT_NONE && !g.scale && g.out_scale == 1.0f && cdiv(g.m, 128) >= 256) {
       p.nch = 1;
       p.ntc = nt;
       return launch_rw<PRO, TA, KS, true>(p, s);

@@ -1707,6 +1707,7 @@ def test_config2_nafnet_gemms(c, h, w, hip_bf16):
     (700, 48, 144, {"ln": True}), (65, 64, 200, {"act": "gelu"}), (97, 32, 32, {"res": "bf16", "scale": True}),
     (200, 48, 56, {"res": "fp32", "out": "fp32", "scale": True}), (130, 96, 264, {"out": "fp32"}),
     (33000, 48, 72, {"ln": True}), (32771, 64, 168, {}),   # tiles stored as one run of memory
+    (33000, 48, 440, {"ln": True}), (33000, 48, 456, {"ln": True}), (32700, 32, 712, {}),  # longest run in LDS, too long
     (33000, 48, 128, {"ln": True})])
 def test_rowwide_kernel(m, k, n, opts, hip_bf16):
     """linear on gemm_rowwide_kernel: remainders of its 32-pixel tiles, 32-channel tiles, 16-k steps and
