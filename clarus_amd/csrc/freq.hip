@@ -1,4 +1,5 @@
-// Per-8x8-patch DFT operators of FFTformer as dense real products on MFMA (gfx950).
+// Per-8x8-patch DFT operators of FFTformer as dense real products on MFMA (gfx950). patch_filter and patch_corr
+// come here only past the 32-bit offsets of fft_patch_kernel, linear_patch_filter with fp32 operands or long K.
 //
 // A patch of one channel is a 64-vector x (pixel r * 8 + s). With the 80 x 64 real matrix
 // Fwd (rows 2b / 2b + 1 = Re / Im of rfft2 bin b = u * 5 + v) and the 64 x 80 matrix Inv
@@ -17,6 +18,7 @@
 
 #include "capi.hpp"
 #include "common.hpp"
+#include "freq_fft.hpp"
 #include "freq_lpf.hpp"
 
 namespace clarus {
@@ -619,6 +621,13 @@ static int launch_patch(FreqP& p, hipStream_t s, const char* what) {
   p.small_offsets = (7 * p.sh + 7 * p.sw + 2 * p.c) < ((int64_t)1 << 31) && p.sh < ((int64_t)1 << 31) &&
                     p.sw < ((int64_t)1 << 31);
   const int64_t patches = p.batch * cdiv(p.h, 8) * cdiv(p.w, 8);
+  // FFTs in registers wherever 32-bit buffer offsets reach (figures at that kernel); the dense products keep the rest
+  if (fft_patch_fits(p.sn, p.sh, p.sw, p.batch, p.h, p.w, p.c, p.corr != 0)) {
+    const FftPatchP q{p.x, p.gain, p.res, p.out, p.sn, p.sh, p.sw, (int)p.h, (int)p.w, (int)p.c, (int)patches,
+                      p.x_dt, p.r_dt, p.o_dt, 0, 0, 0, 0};
+    launch_fft_patch(q, p.corr != 0, s);
+    return check_launch(what);
+  }
   p.units = patches * cdiv(p.c, 16);
   // persistent: 2 resident workgroups per CU (the LDS operator copies), so each stages the
   // matrices once for many units

@@ -337,9 +337,10 @@ int clarus_hip_channel_attention_noalloc(const void* qkv, int32_t qkv_dtype, con
                                          int64_t heads, void* stream);
 
 /*
- * Per 8x8 patch and channel: y = irfft2(rfft2(patch) * g[c]) (+ residual), as the dense
- * real products  y = Inv[64 x 80] . (g_c * (Fwd[80 x 64] . x))  on fp32 MFMA.
- * fwd [80][64] and inv [64][80] fp32 (rows of re/im coefficients, see clarus_amd/dft.py);
+ * Per 8x8 patch and channel: y = irfft2(rfft2(patch) * g[c]) (+ residual), as fp32 FFTs in
+ * registers, which need the gains only, where x and out lie within 2^29 elements; past them as the
+ * dense real products  y = Inv[64 x 80] . (g_c * (Fwd[80 x 64] . x))  with
+ * fwd [80][64] and inv [64][80] fp32, the matrices of rfft2 and irfft2 (clarus_amd/dft.py);
  * gain [c][80] fp32 (the filter per coefficient). x [batch, h, w, c] NHWC with pixel
  * stride ldx; h, w multiples of 8 (the caller reflect-pads other sizes).
  * out [batch, h, w, c] contiguous, dtype o_dtype; residual contiguous like out or NULL.
@@ -376,7 +377,7 @@ int clarus_hip_linear_patch_filter(const void* x, int32_t x_dtype, const void* w
  * FFTformer FSAS correlation (ops/torch_ref.py:278-288): per 8x8 patch,
  * irfft2(rfft2(q) * rfft2(k)) with q = x[..., :c], k = x[..., c:2c]; x has unit channel
  * stride and arbitrary batch / row / pixel strides (elements); out fp32 [batch, h, w, c].
- * fwd [80][64], inv [64][80] as above.
+ * fwd [80][64], inv [64][80] and the two forms as above.
  * replaces kernels/freq.py:165-186 patch_corr
  */
 int clarus_hip_patch_corr(const void* x, int32_t x_dtype, int64_t sn, int64_t sh, int64_t sw,

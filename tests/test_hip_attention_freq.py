@@ -357,3 +357,45 @@ def test_fft_lpf_kernel(h, w, k, n, ln, res, hip_bf16):
     assert _lib.last_kernel().startswith("fft_lpf_kernel"), _lib.last_kernel()
     ref = REF.linear_patch_filter(x, wl, b, f, ln=ln, ln_eps=1e-5, residual=rr)
     assert_bf16(got.cpu(), ref, f"fft lpf {h}x{w} k{k} n{n}")
+
+
+@pytest.mark.parametrize("n,h,w,c,xdt,odt,res", [
+    (1, 8, 8, 1, "fp32", "fp32", None), (2, 13, 21, 33, "bf16", "fp32", "bf16"), (1, 40, 16, 48, "fp32", "bf16", None),
+    (3, 24, 9, 8, "bf16", "bf16", "fp32"), (1, 64, 72, 288, "bf16", "bf16", None), (2, 200, 136, 96, "fp32", "fp32", "fp32"),
+    (1, 5, 6, 40, "fp32", "fp32", "bf16")])
+def test_fft_patch_filter(n, h, w, c, xdt, odt, res, hip_bf16):
+    """patch_filter on fft_patch_kernel: windows of 32 (patch, channel) entries that end within a patch, an image
+    and the batch, reflected edges, a channel slice of a wider tensor, every dtype and residual, against the oracle
+    (24 levels of fp32 butterflies there and here, 2^-25 each: 2e-6 bounds both)
+    (gains without the symmetry of a real filter's spectrum in columns 0 and 4)."""
+    from clarus_amd import _lib
+    g = gen(h + w + c)
+    dts = {"fp32": torch.float32, "bf16": torch.bfloat16}
+    wide, f = rnd(g, n, h, w, c + 8, dtype=dts[xdt]), rnd(g, c, 8, 5)
+    rr = rnd(g, n, h, w, c, dtype=dts[res]) if res else None
+    got = hip_bf16.patch_filter(wide.cuda()[..., 8:], f.cuda(), residual=None if rr is None else rr.cuda(), out_dtype=dts[odt])
+    assert _lib.last_kernel().startswith("fft_patch_kernel"), _lib.last_kernel()
+    ref = REF.patch_filter(wide[..., 8:], f, residual=rr, out_dtype=torch.float32)
+    if odt == "fp32":
+        assert_fp32(got.cpu(), ref, rel=2e-6, what=f"fft patch_filter {n}x{h}x{w}x{c}")
+    else:
+        assert_bf16(got.cpu(), ref, f"fft patch_filter {n}x{h}x{w}x{c}")
+
+
+@pytest.mark.parametrize("n,h,w,c", [(1, 8, 8, 1), (2, 16, 24, 33), (3, 40, 8, 48), (1, 96, 128, 96), (2, 64, 64, 40)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_fft_patch_corr(n, h, w, c, dt, hip_bf16, hip_f32):
+    """patch_corr on fft_patch_kernel, q and k slices of a wider tensor, against the oracle; and the dense-product
+    form, which takes what lies past 32-bit offsets (here a batch stride that one image never steps)."""
+    from clarus_amd import _lib
+    g = gen(h + w + c)
+    x = rnd(g, n, h, w, 3 * c + 1, dtype=dt)
+    hip, xd = hip_bf16 if dt == torch.bfloat16 else hip_f32, x.cuda()
+    got = hip.patch_corr(xd, c)
+    assert _lib.last_kernel().startswith("fft_patch_kernel corr=1"), _lib.last_kernel()
+    ref = REF.patch_corr(x, c)
+    assert_fp32(got.cpu(), ref, rel=2e-6, what=f"fft patch_corr {n}x{h}x{w}x{c}")
+    one = xd[:1].as_strided((1, h, w, 3 * c + 1), (1 << 31, *xd.stride()[1:]))
+    dense = hip.patch_corr(one, c)
+    assert _lib.last_kernel().startswith("patch_kernel corr=1"), _lib.last_kernel()
+    assert_fp32(dense.cpu(), ref[:1], rel=1e-5, what=f"dense patch_corr {h}x{w}x{c}")
