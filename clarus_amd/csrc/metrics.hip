@@ -13,8 +13,8 @@
 // Kernels (all sums in a fixed order: deterministic):
 //   ssd_max_kernel   per-workgroup int64 sum of squared differences and max(pred) partials
 //   ssim_tile_kernel 8 x 32 output pixels x 3 channels per workgroup: the u8 tiles with a
-//                    5-pixel clamped halo in LDS, channel mix + horizontal pass into LDS (fp64),
-//                    vertical pass and the SSIM map for both constant sets (max(pred) <= 1 or
+//                    5-pixel clamped halo in LDS, horizontal pass into LDS (fp64), vertical pass,
+//                    channel mix and the SSIM map for both constant sets (max(pred) <= 1 or
 //                    not, decided later), per-workgroup sums
 //   finish_kernel    one workgroup: the partials in order -> res[0] = PSNR, res[1] = SSIM
 // replaces python/clarus/metrics.py:59-159 (ssd_max_kernel, ssim_h_kernel, ssim_v_kernel) and
@@ -43,6 +43,7 @@ struct MetricsP {
   double* res;             // [2]
   int64_t h, w, n;         // n = h w 3
   int64_t nb, nt;
+  double g[11], cm[9];     // the normalised 11-tap Gaussian (sigma 1.5) and the channel-mixing matrix
 };
 
 __global__ void __launch_bounds__(SS_BLOCK) ssd_max_kernel(const MetricsP p) {
@@ -88,35 +89,22 @@ __global__ void __launch_bounds__(SS_BLOCK) ssd_max_kernel(const MetricsP p) {
   }
 }
 
-// the normalised 11-tap Gaussian (sigma 1.5) in fp64, and the channel-mixing matrix
-__device__ void gauss_tables(double* g, double* cm) {
-  if (threadIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < 11; ++i) {
-      g[i] = exp(-(double)((i - 5) * (i - 5)) / (2.0 * 1.5 * 1.5));
-      s += g[i];
-    }
-    for (int i = 0; i < 11; ++i) g[i] /= s;
-    for (int c = 0; c < 9; ++c) cm[c] = 0.0;
-    for (int c = 0; c < 3; ++c)
-      for (int t = -5; t <= 5; ++t) {
-        int cc = c + t;
-        cc = cc < 0 ? 0 : (cc > 2 ? 2 : cc);
-        cm[c * 3 + cc] += g[t + 5];
-      }
-  }
-}
+// Bound: fp64 FMAs (about 195 per output value: 11 taps x 5 moments, twice 2.25 for the halo rows and once, and 15
+// for the mix) and the LDS reads of the vertical pass. The taps come as kernel arguments (scalar registers: one thread
+// of every workgroup evaluating 11 fp64 exponentials first, and a tap read from LDS per FMA, were a large part of the
+// time); the three linear passes commute, so the channel mix runs last, on one pixel's three channels in a thread, not
+// on every pixel of the halo. Horizontal results: one plane per moment and channel, rows of 33 values, so that the
+// writes (16 rows x 4 runs per wave) and the reads (32 columns) fall on distinct banks.
+constexpr int HM_ROW = MT_W + 1;
 
 __global__ void __launch_bounds__(256) ssim_tile_kernel(const MetricsP p) {
   __shared__ unsigned char ta[MT_RH][MT_RW][3], tb[MT_RH][MT_RW][3];
-  __shared__ double hm[5][MT_RH][MT_W][3];  // mixed + horizontally filtered a, b, a^2, b^2, ab
-  __shared__ double g[11], cm[9];
-  __shared__ double red[2][256];
+  __shared__ double hm[5][3][MT_RH][HM_ROW];  // horizontally filtered a, b, a^2, b^2, ab
+  __shared__ double red[2][4];
   const int H = (int)p.h, W = (int)p.w;
   const int tiles_x = (W + MT_W - 1) / MT_W;
   const int ty = blockIdx.x / tiles_x, tx = blockIdx.x - ty * tiles_x;
   const int y0 = ty * MT_H, x0 = tx * MT_W;
-  gauss_tables(g, cm);
   // u8 tiles with a clamped (replicate) halo
   for (int e = threadIdx.x; e < MT_RH * MT_RW; e += 256) {
     const int r = e / MT_RW, c = e - r * MT_RW;
@@ -131,73 +119,76 @@ __global__ void __launch_bounds__(256) ssim_tile_kernel(const MetricsP p) {
     }
   }
   __syncthreads();
-  // channel mix + horizontal pass, moments about 128. A thread takes a run of HR consecutive
-  // output columns of one (row, channel): it mixes the HR + 10 pixels its windows span once per
-  // moment (in registers) and slides the 11 taps over them, instead of mixing every tap's pixel
-  // again for each output (11 times the mixing work). Per output the same sums in the same order.
+  // horizontal pass, moments about 128 (exact integers): a thread takes a run of HR consecutive output columns of
+  // one (row, channel) and slides the 11 taps over the HR + 10 pixels its windows span
   constexpr int HR = 8, HRUNS = MT_W / HR;
   static_assert(MT_W % HR == 0 && MT_RH * 3 * HRUNS <= 256, "one run per thread");
   if ((int)threadIdx.x < MT_RH * 3 * HRUNS) {
-    const int e = threadIdx.x;
-    const int r = e / (3 * HRUNS), rem = e - r * (3 * HRUNS), k = rem / HRUNS, c0 = (rem - k * HRUNS) * HR;
-    const double w0 = cm[k * 3], w1 = cm[k * 3 + 1], w2 = cm[k * 3 + 2];
+    const int e = threadIdx.x / HRUNS, c0 = (threadIdx.x % HRUNS) * HR;
+    const int k = e / MT_RH, r = e - k * MT_RH;
+    int av[HR + 10], bv[HR + 10];
+#pragma unroll
+    for (int j = 0; j < HR + 10; ++j) {
+      av[j] = (int)ta[r][c0 + j][k] - 128;
+      bv[j] = (int)tb[r][c0 + j][k] - 128;
+    }
 #pragma unroll
     for (int q = 0; q < 5; ++q) {
       double m[HR + 10];
 #pragma unroll
-      for (int j = 0; j < HR + 10; ++j) {
-        double mq = 0.0;
-#pragma unroll
-        for (int kk = 0; kk < 3; ++kk) {
-          const double wgt = kk == 0 ? w0 : (kk == 1 ? w1 : w2);
-          const double av = (double)ta[r][c0 + j][kk] - 128.0, bv = (double)tb[r][c0 + j][kk] - 128.0;
-          if (q == 0) mq += wgt * av;
-          else if (q == 1) mq += wgt * bv;
-          else if (q == 2) mq += wgt * av * av;
-          else if (q == 3) mq += wgt * bv * bv;
-          else mq += wgt * av * bv;
-        }
-        m[j] = mq;
-      }
+      for (int j = 0; j < HR + 10; ++j)
+        m[j] = (double)(q == 0 ? av[j] : q == 1 ? bv[j] : q == 2 ? av[j] * av[j] : q == 3 ? bv[j] * bv[j] : av[j] * bv[j]);
 #pragma unroll
       for (int i = 0; i < HR; ++i) {
         double sq = 0.0;
 #pragma unroll
-        for (int t = 0; t < 11; ++t) sq += g[t] * m[i + t];
-        hm[q][r][c0 + i][k] = sq;
+        for (int t = 0; t < 11; ++t) sq += p.g[t] * m[i + t];
+        hm[q][k][r][c0 + i] = sq;
       }
     }
   }
   __syncthreads();
-  // vertical pass and the SSIM map, both constant sets
+  // vertical pass of one pixel's channels, channel mix and the SSIM map, both constant sets
+  static_assert(MT_H * MT_W == 256, "one pixel per thread");
   double sum_lo = 0.0, sum_hi = 0.0;
   const double c1l = 0.01 * 0.01, c2l = 0.03 * 0.03, c1h = (0.01 * 255) * (0.01 * 255), c2h = (0.03 * 255) * (0.03 * 255);
-  for (int e = threadIdx.x; e < MT_H * MT_W * 3; e += 256) {
-    const int r = e / (MT_W * 3), rem = e - r * (MT_W * 3), c = rem / 3, k = rem - (rem / 3) * 3;
-    if (y0 + r >= H || x0 + c >= W) continue;
-    double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int t = 0; t < 11; ++t)
+  const int r = (int)threadIdx.x / MT_W, c = (int)threadIdx.x % MT_W;
+  if (y0 + r < H && x0 + c < W) {
+    double v[3][5];
 #pragma unroll
-      for (int q = 0; q < 5; ++q) v[q] += g[t] * hm[q][r + t][c][k];
-    const double s11 = v[2] - v[0] * v[0], s22 = v[3] - v[1] * v[1], s12 = v[4] - v[0] * v[1];
-    const double mu1 = v[0] + 128.0, mu2 = v[1] + 128.0;
-    const double m12 = mu1 * mu2, msq = mu1 * mu1 + mu2 * mu2;
-    sum_lo += ((2.0 * m12 + c1l) * (2.0 * s12 + c2l)) / ((msq + c1l) * (s11 + s22 + c2l));
-    sum_hi += ((2.0 * m12 + c1h) * (2.0 * s12 + c2h)) / ((msq + c1h) * (s11 + s22 + c2h));
-  }
-  red[0][threadIdx.x] = sum_lo;
-  red[1][threadIdx.x] = sum_hi;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      red[0][threadIdx.x] += red[0][threadIdx.x + o];
-      red[1][threadIdx.x] += red[1][threadIdx.x + o];
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int q = 0; q < 5; ++q) {
+        double s = 0.0;
+#pragma unroll
+        for (int t = 0; t < 11; ++t) s += p.g[t] * hm[q][k][r + t][c];
+        v[k][q] = s;
+      }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      double x[5];
+#pragma unroll
+      for (int q = 0; q < 5; ++q) x[q] = p.cm[3 * k] * v[0][q] + p.cm[3 * k + 1] * v[1][q] + p.cm[3 * k + 2] * v[2][q];
+      const double s11 = x[2] - x[0] * x[0], s22 = x[3] - x[1] * x[1], s12 = x[4] - x[0] * x[1];
+      const double mu1 = x[0] + 128.0, mu2 = x[1] + 128.0;
+      const double m12 = mu1 * mu2, msq = mu1 * mu1 + mu2 * mu2;
+      sum_lo += ((2.0 * m12 + c1l) * (2.0 * s12 + c2l)) / ((msq + c1l) * (s11 + s22 + c2l));
+      sum_hi += ((2.0 * m12 + c1h) * (2.0 * s12 + c2h)) / ((msq + c1h) * (s11 + s22 + c2h));
     }
-    __syncthreads();
   }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    sum_lo += __shfl_xor(sum_lo, o, 64);
+    sum_hi += __shfl_xor(sum_hi, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = sum_lo;
+    red[1][threadIdx.x >> 6] = sum_hi;
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
-    p.ssim[2 * blockIdx.x] = red[0][0];
-    p.ssim[2 * blockIdx.x + 1] = red[1][0];
+    p.ssim[2 * blockIdx.x] = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+    p.ssim[2 * blockIdx.x + 1] = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
   }
 }
 
@@ -239,6 +230,22 @@ __global__ void __launch_bounds__(256) finish_kernel(const MetricsP p) {
   }
 }
 
+void gauss_tables(double* g, double* cm) {
+  double s = 0.0;
+  for (int i = 0; i < 11; ++i) {
+    g[i] = exp(-(double)((i - 5) * (i - 5)) / (2.0 * 1.5 * 1.5));
+    s += g[i];
+  }
+  for (int i = 0; i < 11; ++i) g[i] /= s;
+  for (int c = 0; c < 9; ++c) cm[c] = 0.0;
+  for (int c = 0; c < 3; ++c)
+    for (int t = -5; t <= 5; ++t) {
+      int cc = c + t;
+      cc = cc < 0 ? 0 : (cc > 2 ? 2 : cc);
+      cm[c * 3 + cc] += g[t + 5];
+    }
+}
+
 void metrics_layout(int64_t h, int64_t w, int64_t& nb, int64_t& nt) {
   nb = cdiv(h * w * 3, SS_CHUNK);
   nt = cdiv(h, MT_H) * cdiv(w, MT_W);
@@ -271,6 +278,7 @@ extern "C" int clarus_hip_psnr_ssim(const void* pred, const void* gt, int64_t h,
   p.b = (const unsigned char*)gt;
   p.h = h; p.w = w; p.n = h * w * 3;
   metrics_layout(h, w, p.nb, p.nt);
+  gauss_tables(p.g, p.cm);
   unsigned char* s = (unsigned char*)scratch;
   p.ssd = (long long*)s;
   p.mx = (int*)(s + p.nb * 8);
