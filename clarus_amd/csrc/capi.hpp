@@ -2,6 +2,8 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <atomic>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -40,5 +42,19 @@ inline int check_launch(const char* what) {
       return CLARUS_EINVAL;         \
     }                               \
   } while (0)
+
+// workgroups of a kernel that fit a CU, kept for the last (threads, dynamic LDS) asked of this kernel: the runtime's
+// query is host work on every launch otherwise
+struct OccupancyMemo {
+  std::atomic<uint64_t> last{0};  // workgroups (16 bits) | threads (16) | LDS bytes (32); 0: nothing asked yet
+  int get(const void* fn, int threads, int lds) {
+    const uint64_t key = (uint64_t)(uint16_t)threads << 32 | (uint32_t)lds, v = last.load(std::memory_order_relaxed);
+    if (v >> 48 && (v & 0xffffffffffffull) == key) return (int)(v >> 48);
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, threads, lds) != hipSuccess || n < 1) n = 1;
+    last.store((uint64_t)n << 48 | key, std::memory_order_relaxed);
+    return n;
+  }
+};
 
 }  // namespace clarus

@@ -256,10 +256,8 @@ void launch_fp(FftPatchP& p, hipStream_t s) {
   // a workgroup: whole groups of up to 8 waves, so the 128-byte lines that windows share stay in one CU
   const int waves = p.windows <= 8 ? 8 / p.windows * p.windows : 8;
   auto fn = &fft_patch_kernel<XDT, CORR, EDGE>;
-  int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(fn), 64 * waves, 0) != hipSuccess ||
-      per_cu < 1)
-    per_cu = 1;
+  static OccupancyMemo occ;
+  const int per_cu = occ.get(reinterpret_cast<const void*>(fn), 64 * waves, 0);
   // as many streams of groups as whole workgroups hold, up to the waves that run at once
   const int64_t cap = std::max<int64_t>(1, (int64_t)device_cus() * per_cu * waves / p.windows);
   p.streams = (int)std::min<int64_t>(p.groups, cap);

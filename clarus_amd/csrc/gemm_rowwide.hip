@@ -312,10 +312,8 @@ void launch_rw(RwP& p, hipStream_t s) {
   (void)set;
   const GemmP& g = p.g;
   const int lds = rw_lds<KS, LIN>(p.ntc, (int)g.n);
-  int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(fn), 256, lds) != hipSuccess ||
-      per_cu < 1)
-    per_cu = 1;
+  static OccupancyMemo occ;
+  const int per_cu = occ.get(reinterpret_cast<const void*>(fn), 256, lds);
   const int64_t cap = std::max<int64_t>(1, (int64_t)device_cus() * per_cu / (8 * p.nch));
   const int64_t groups = std::min<int64_t>(cdiv(cdiv(g.m, 32), 4 * 8), cap);  // workgroups per XCD and chunk
   note_kernel("gemm_rowwide_kernel pro=%d a=%s ks=%d tiles=%d chunks=%d lin=%d", g.pro, TA == DT_BF16 ? "bf16" : "f32",
