@@ -97,6 +97,8 @@ SIGNATURES = {
     "clarus_hip_last_error": (ctypes.c_char_p, []),
     "clarus_hip_last_kernel": (ctypes.c_char_p, []),
 }
+for _name in ("patch_filter", "patch_corr", "linear_patch_filter"):
+    SIGNATURES[f"clarus_hip_{_name}_rfft2"] = SIGNATURES[f"clarus_hip_{_name}"]
 
 _LIB = None
 

@@ -1,5 +1,6 @@
-// Per-8x8-patch DFT operators of FFTformer as dense real products on MFMA (gfx950). patch_filter and patch_corr
-// come here only past the 32-bit offsets of fft_patch_kernel, linear_patch_filter with fp32 operands or long K.
+// Per-8x8-patch DFT operators of FFTformer as dense real products on MFMA (gfx950): what the caller's matrices say.
+// The _rfft2 entries, whose transforms are rfft2 / irfft2, come here only past the 32-bit offsets of
+// fft_patch_kernel and with fp32 operands or long K in linear_patch_filter.
 //
 // A patch of one channel is a 64-vector x (pixel r * 8 + s). With the 80 x 64 real matrix
 // Fwd (rows 2b / 2b + 1 = Re / Im of rfft2 bin b = u * 5 + v) and the 64 x 80 matrix Inv
@@ -391,10 +392,20 @@ struct LpfP {
   int r_dt, o_dt;
 };
 
-template <int XDT, int LN, bool WS, int CB, int KS>
+// W^T rows held in LDS (bf16 weights, N K 2 bytes at most this many): two workgroups per CU still fit
+constexpr int LPF_WL_MAX = 30 * 1024;
+
+// WL: the bf16 W^T [n][k] is copied into (dynamic) LDS once per workgroup and read from there.
+template <int XDT, int LN, bool WS, int CB, int KS, bool WL>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) lpf_kernel(const LpfP p) {
   __shared__ __attribute__((aligned(16))) unsigned char fw[2 * FBYTES];  // Fwd hi, lo (columns permuted)
   __shared__ __attribute__((aligned(16))) unsigned char iv[2 * IBYTES];
+  extern __shared__ __attribute__((aligned(16))) unsigned char wls[];    // W^T [n][k] bf16 (WL)
+  if constexpr (WL) {
+    const int nu = (int)(p.n * p.k / 8);  // 16-byte units
+    for (int e = threadIdx.x; e < nu; e += 256)
+      *reinterpret_cast<u32x4*>(wls + e * 16) = reinterpret_cast<const u32x4*>(p.wt)[e];
+  }
   for (int e = threadIdx.x; e < NCOEF * 16; e += 256) {  // Fwd [80][64] in the GEMM's pixel order
     const int r = e >> 4, c4 = (e & 15) * 4;             // staged columns c4 .. c4 + 3
     const int kb = c4 >> 5, lgs = (c4 >> 3) & 3, i0 = c4 & 7;  // i0 = 0 or 4
@@ -409,20 +420,31 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) l
   constexpr int XES = XDT == DT_BF16 ? 2 : 4;
   constexpr int WES = WS ? 4 : 2;
   constexpr int MAXS = KS;                              // LN rows in registers: K <= 32 KS
+  // patch-major order (LayerNorm rows normalised once per patch, held as hi + lo bf16 fragments
+  // through all channel tiles) for bf16 weights and K <= 96
+  constexpr bool PM = LN != 0 && !WS && KS <= 3;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lc = lane & 15, lg = lane >> 4;
   const int H = (int)p.h, W = (int)p.w, K = (int)p.k;
   const int ph = (int)cdiv(p.h, 8), pw = (int)cdiv(p.w, 8);
   const int ctiles = (int)cdiv(p.n, 16 * CB);  // channel tiles of CB 16-channel blocks
+  // 8 bf16 weights of a W^T row at k0: from the LDS copy (WL) or global memory
   auto wload = [&](const unsigned char* row, int k0) __attribute__((always_inline)) -> bf16x8 {
-    return *reinterpret_cast<const bf16x8*>(row + (int64_t)k0 * 2);
+    if constexpr (WL) {
+      const int off = (int)(row - wls) + k0 * 2;
+      return *reinterpret_cast<const bf16x8*>(wls + off);
+    } else {
+      return *reinterpret_cast<const bf16x8*>(row + (int64_t)k0 * 2);
+    }
   };
   const int S = (int)cdiv(p.k, 32);            // 32-k steps
   const float invk = 1.0f / (float)K;
 
   // forward DFT, gains, inverse, + residual, store of one channel tile (GEMM outputs dd, + bias)
+  // (lc, lg passed in: the patch-major loop hands over copies it re-derives per channel tile, so
+  // the per-lane addresses built from them are not held across the loop)
   auto finish = [&](f32x4 (&dd)[CB][4], const int64_t (&chl)[CB], const bool (&cval)[CB], const int64_t n,
-                    const int py, const int px) __attribute__((always_inline)) {
+                    const int py, const int px, const int lc, const int lg) __attribute__((always_inline)) {
       // ---- forward DFT: B operand k-block kb = pixel blocks 2 kb (slots 0-3), 2 kb + 1 (4-7); each
       // operator fragment read from LDS once for the CB blocks
       bf16x8 xh[CB][2], xl[CB][2];
@@ -511,6 +533,91 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) l
       }
   };
 
+  if constexpr (PM) {
+    // one wave per patch: its 64 rows normalised once, held as MFMA A fragments (hi + lo bf16
+    // pairs) through all channel tiles of the patch
+    const int64_t npatch = p.batch * ph * pw;
+    for (int64_t pt = (int64_t)blockIdx.x * 4 + wave; pt < npatch; pt += (int64_t)gridDim.x * 4) {
+      asm volatile("" ::: "memory");
+      const int64_t n = pt / ((int64_t)ph * pw);
+      const int rem = (int)(pt - n * ph * pw);
+      const int py = rem / pw, px = rem - (rem / pw) * pw;
+      bf16x8 ah[4][KS], al[4][KS];
+#pragma unroll
+      for (int pb = 0; pb < 4; ++pb) {
+        const int pp = pb * 16 + lc;  // this lane's A row: patch pixel pp
+        int yy = py * 8 + (pp >> 3), xx = px * 8 + (pp & 7);
+        if (yy >= H) yy = 2 * (H - 1) - yy;
+        if (xx >= W) xx = 2 * (W - 1) - xx;
+        const unsigned char* arow = (const unsigned char*)p.x + (((n * H + yy) * W + xx) * p.k) * XES;
+        f32x8 a[KS];
+        float s1 = 0.f;
+#pragma unroll
+        for (int st = 0; st < KS; ++st) {
+          const int k0 = st * 32 + lg * 8;
+          a[st] = (st < S && k0 < K) ? load8<XDT>(arow + (int64_t)k0 * XES) : zero8();
+#pragma unroll
+          for (int i = 0; i < 8; ++i) s1 += a[st].v[i];
+        }
+        const float mean = LN == 1 ? sum_col4(s1) * invk : 0.f;
+        float s2 = 0.f;
+#pragma unroll
+        for (int st = 0; st < KS; ++st) {
+          const bool kv = st < S && st * 32 + lg * 8 < K;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const float d = kv ? a[st].v[i] - mean : 0.f;
+            s2 += d * d;
+          }
+        }
+        const float rstd = rsqrtf(sum_col4(s2) * invk + p.eps);
+#pragma unroll
+        for (int st = 0; st < KS; ++st) {
+          const bool kv = st < S && st * 32 + lg * 8 < K;
+          f32x8 v;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) v.v[i] = kv ? (a[st].v[i] - mean) * rstd : 0.f;
+          split_bf16(v, ah[pb][st], al[pb][st]);
+        }
+      }
+#pragma unroll 1
+      for (int ct = 0; ct < ctiles; ++ct) {
+        asm volatile("" ::: "memory");
+        int lc = lane & 15, lg = lane >> 4;
+        asm volatile("" : "+v"(lc), "+v"(lg));
+        int64_t chl[CB];
+        bool cval[CB];
+        const unsigned char* wrow[CB];
+        f32x4 dd[CB][4];
+#pragma unroll
+        for (int b = 0; b < CB; ++b) {
+          const int64_t ch = ((int64_t)ct * CB + b) * 16 + lc;
+          cval[b] = ch < p.n;
+          chl[b] = cval[b] ? ch : 0;
+          wrow[b] = WL ? wls + chl[b] * p.k * 2 : (const unsigned char*)p.wt + chl[b] * p.k * WES;
+          const float bv = (cval[b] && p.bias) ? p.bias[chl[b]] : 0.f;
+#pragma unroll
+          for (int pb = 0; pb < 4; ++pb) dd[b][pb] = f32x4{bv, bv, bv, bv};
+        }
+#pragma unroll
+        for (int st = 0; st < KS; ++st) {
+          if (st >= S) continue;
+          const int k0 = st * 32 + lg * 8;
+          const bool kv = k0 < K;
+#pragma unroll
+          for (int b = 0; b < CB; ++b) {
+            const bf16x8 wv = (cval[b] && kv) ? wload(wrow[b], k0) : bf16x8{};
+#pragma unroll
+            for (int pb = 0; pb < 4; ++pb) {
+              dd[b][pb] = mfma_bf16(ah[pb][st], wv, dd[b][pb]);
+              dd[b][pb] = mfma_bf16(al[pb][st], wv, dd[b][pb]);
+            }
+          }
+        }
+        finish(dd, chl, cval, n, py, px, lc, lg);
+      }
+    }
+  } else {
   for (int64_t u = (int64_t)blockIdx.x * 4 + wave; u < p.units; u += (int64_t)gridDim.x * 4) {
       asm volatile("" ::: "memory");
       const int ct = (int)(u % ctiles);
@@ -527,7 +634,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) l
         const int64_t ch = ((int64_t)ct * CB + b) * 16 + lc;
         cval[b] = ch < p.n;
         chl[b] = cval[b] ? ch : 0;
-        wrow[b] = (const unsigned char*)p.wt + chl[b] * p.k * WES;
+        wrow[b] = WL ? wls + chl[b] * p.k * 2 : (const unsigned char*)p.wt + chl[b] * p.k * WES;
         bias[b] = (cval[b] && p.bias) ? p.bias[chl[b]] : 0.f;
       }
 
@@ -613,16 +720,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) l
         }
       }
 
-      finish(dd, chl, cval, n, py, px);
+      finish(dd, chl, cval, n, py, px, lc, lg);
     }
+  }
 }
 
-static int launch_patch(FreqP& p, hipStream_t s, const char* what) {
+// rfft2: the transforms are rfft2 / irfft2 (fwd and inv their matrices), so FFTs may compute them
+static int launch_patch(FreqP& p, bool rfft2, hipStream_t s, const char* what) {
   p.small_offsets = (7 * p.sh + 7 * p.sw + 2 * p.c) < ((int64_t)1 << 31) && p.sh < ((int64_t)1 << 31) &&
                     p.sw < ((int64_t)1 << 31);
   const int64_t patches = p.batch * cdiv(p.h, 8) * cdiv(p.w, 8);
   // FFTs in registers wherever 32-bit buffer offsets reach (figures at that kernel); the dense products keep the rest
-  if (fft_patch_fits(p.sn, p.sh, p.sw, p.batch, p.h, p.w, p.c, p.corr != 0)) {
+  if (rfft2 && fft_patch_fits(p.sn, p.sh, p.sw, p.batch, p.h, p.w, p.c, p.corr != 0)) {
     const FftPatchP q{p.x, p.gain, p.res, p.out, p.sn, p.sh, p.sw, (int)p.h, (int)p.w, (int)p.c, (int)patches,
                       p.x_dt, p.r_dt, p.o_dt, 0, 0, 0, 0};
     launch_fft_patch(q, p.corr != 0, s);
@@ -646,14 +755,9 @@ static int launch_patch(FreqP& p, hipStream_t s, const char* what) {
   return check_launch(what);
 }
 
-}  // namespace clarus
-
-using namespace clarus;
-
-extern "C" int clarus_hip_patch_filter(const void* x, int32_t x_dtype, int64_t ldx, const float* fwd,
-                                       const float* inv, const float* gain, const void* res, int32_t r_dtype,
-                                       void* out, int32_t o_dtype, int64_t batch, int64_t h, int64_t w, int64_t c,
-                                       void* stream) {
+static int run_patch_filter(bool rfft2, const void* x, int32_t x_dtype, int64_t ldx, const float* fwd, const float* inv,
+                            const float* gain, const void* res, int32_t r_dtype, void* out, int32_t o_dtype,
+                            int64_t batch, int64_t h, int64_t w, int64_t c, void* stream) {
   clear_error();
   CLARUS_REQUIRE(x && fwd && inv && gain && out, "patch_filter: null operand");
   CLARUS_REQUIRE(batch > 0 && h > 0 && w > 0 && c > 0 && ldx >= c, "patch_filter: bad sizes");
@@ -668,12 +772,11 @@ extern "C" int clarus_hip_patch_filter(const void* x, int32_t x_dtype, int64_t l
   p.sn = h * w * ldx; p.sh = w * ldx; p.sw = ldx;
   p.batch = batch; p.h = h; p.w = w; p.c = c;
   p.x_dt = x_dtype; p.r_dt = r_dtype; p.o_dt = o_dtype; p.corr = 0;
-  return launch_patch(p, (hipStream_t)stream, "patch_filter");
+  return launch_patch(p, rfft2, (hipStream_t)stream, "patch_filter");
 }
 
-extern "C" int clarus_hip_patch_corr(const void* x, int32_t x_dtype, int64_t sn, int64_t sh, int64_t sw,
-                                     const float* fwd, const float* inv, float* out, int64_t batch, int64_t h,
-                                     int64_t w, int64_t c, void* stream) {
+static int run_patch_corr(bool rfft2, const void* x, int32_t x_dtype, int64_t sn, int64_t sh, int64_t sw, const float* fwd,
+                          const float* inv, float* out, int64_t batch, int64_t h, int64_t w, int64_t c, void* stream) {
   clear_error();
   CLARUS_REQUIRE(x && fwd && inv && out, "patch_corr: null operand");
   CLARUS_REQUIRE(batch > 0 && h > 0 && w > 0 && c > 0 && h % 8 == 0 && w % 8 == 0,
@@ -685,14 +788,18 @@ extern "C" int clarus_hip_patch_corr(const void* x, int32_t x_dtype, int64_t sn,
   p.sn = sn; p.sh = sh; p.sw = sw;
   p.batch = batch; p.h = h; p.w = w; p.c = c;
   p.x_dt = x_dtype; p.r_dt = DT_F32; p.o_dt = DT_F32; p.corr = 1;
-  return launch_patch(p, (hipStream_t)stream, "patch_corr");
+  return launch_patch(p, rfft2, (hipStream_t)stream, "patch_corr");
 }
 
-extern "C" int clarus_hip_linear_patch_filter(const void* x, int32_t x_dtype, const void* wt, int32_t w_dtype,
-                                              const float* bias, int32_t ln, float ln_eps, const float* fwd,
-                                              const float* inv, const float* gain, const void* res, int32_t r_dtype,
-                                              void* out, int32_t o_dtype, int64_t batch, int64_t h, int64_t w,
-                                              int64_t k, int64_t n, void* stream) {
+// dynamic LDS beyond the default 64 KiB per workgroup (static operators + the W^T copy)
+static void lpf_allow_lds(const void* fn) {
+  (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, LPF_WL_MAX);
+}
+
+static int run_linear_patch_filter(bool rfft2, const void* x, int32_t x_dtype, const void* wt, int32_t w_dtype,
+                                   const float* bias, int32_t ln, float ln_eps, const float* fwd, const float* inv,
+                                   const float* gain, const void* res, int32_t r_dtype, void* out, int32_t o_dtype,
+                                   int64_t batch, int64_t h, int64_t w, int64_t k, int64_t n, void* stream) {
   clear_error();
   CLARUS_REQUIRE(x && wt && fwd && inv && gain && out, "linear_patch_filter: null operand");
   CLARUS_REQUIRE(batch > 0 && h > 0 && w > 0 && k > 0 && n > 0, "linear_patch_filter: bad sizes");
@@ -713,7 +820,8 @@ extern "C" int clarus_hip_linear_patch_filter(const void* x, int32_t x_dtype, co
   // bf16 rows and weights with K <= 96 (with a prologue) or 192: the FFT form, faster at every size measured
   // (figures at its kernel); the dense-product kernel below keeps fp32 operands, longer K and patch rows past
   // 32-bit offsets
-  if (x_dtype == DT_BF16 && w_dtype == DT_BF16 && h < (1 << 30) && w < (1 << 30) && k < (1 << 20) && n < (1 << 24)) {
+  if (rfft2 && x_dtype == DT_BF16 && w_dtype == DT_BF16 && h < (1 << 30) && w < (1 << 30) && k < (1 << 20) &&
+      n < (1 << 24)) {
     LpfFftP q{x, wt, bias, gain, res, out, batch * cdiv(h, 8) * cdiv(w, 8), (int)h, (int)w, (int)k, (int)n, ln_eps,
               (int)(ln == 2), r_dtype, o_dtype};
     if (launch_lpf_fft(q, ln != 0, (hipStream_t)stream)) return check_launch("linear_patch_filter");
@@ -721,12 +829,15 @@ extern "C" int clarus_hip_linear_patch_filter(const void* x, int32_t x_dtype, co
   // channel tile: 2 16-channel blocks of one patch per wave (operator fragments and A rows reused
   // twice; 3 blocks hold ~230 VGPRs, one wave per SIMD, and ran 1.19 against 0.96 ms at the
   // FFTformer level-0 DFFN shape). With a LayerNorm / RMS prologue the row is held in KS 32-k
-  // steps, the fewest that cover K.
+  // steps, the fewest that cover K. bf16 W^T of at most LPF_WL_MAX bytes is read from LDS.
   const int cb = 2;
+  const bool wl = w_dtype == DT_BF16 && n * k * 2 <= LPF_WL_MAX;
+  const size_t wl_bytes = wl ? (size_t)(n * k * 2) : 0;
   const int steps = (int)cdiv(k, 32);
-  const int ks = steps <= 2 && w_dtype == DT_F32 ? 2 : steps <= 3 && w_dtype == DT_F32 ? 3 : steps <= 4 ? 4 : steps <= 6 ? 6 : 8;
+  const int ks = steps <= 2 ? 2 : steps <= 3 ? 3 : steps <= 4 ? 4 : steps <= 6 ? 6 : 8;
   p.units = batch * cdiv(h, 8) * cdiv(w, 8) * cdiv(n, 16 * cb);
-  // persistent: 2 resident workgroups per CU (the two-block tile holds ~170 VGPRs: 2 waves per SIMD)
+  // persistent: 2 resident workgroups per CU (the two-block tile holds ~170 VGPRs: 2 waves per
+  // SIMD; the operators and a W^T copy take ~76 KiB of LDS)
   int64_t blocks = cdiv(p.units, 4);
   if (blocks > 2LL * device_cus()) blocks = 2LL * device_cus();
   const dim3 g((unsigned)blocks);
@@ -737,18 +848,27 @@ extern "C" int clarus_hip_linear_patch_filter(const void* x, int32_t x_dtype, co
   const bool same = (x_dtype == DT_BF16) == (w_dtype == DT_BF16);
   CLARUS_REQUIRE(ln == 0 || same, "linear_patch_filter: a LayerNorm / RMS prologue needs activations and weights "
                  "of one dtype");
-  note_kernel("lpf_kernel ln=%d ws=%d cb=%d ks=%d", ln, w_dtype == DT_F32, cb, ln ? ks : 0);
-#define CLARUS_LPF_CB(XDT, LNV, WSV, KSV) \
-  hipLaunchKernelGGL((lpf_kernel<XDT, LNV, WSV, 2, KSV>), g, dim3(256), 0, s, p)
-#define CLARUS_LPF_KS(XDT, LNV, WSV)                                     \
-  do {                                                                   \
-    switch (ks) {                                                        \
-      case 2: CLARUS_LPF_CB(XDT, LNV, WSV, (WSV ? 2 : 4)); break;        \
-      case 3: CLARUS_LPF_CB(XDT, LNV, WSV, (WSV ? 3 : 4)); break;        \
-      case 4: CLARUS_LPF_CB(XDT, LNV, WSV, 4); break;                    \
-      case 6: CLARUS_LPF_CB(XDT, LNV, WSV, 6); break;                    \
-      default: CLARUS_LPF_CB(XDT, LNV, WSV, 8); break;                   \
-    }                                                                    \
+  note_kernel("lpf_kernel ln=%d ws=%d cb=%d ks=%d wl=%d", ln, w_dtype == DT_F32, cb, ln ? ks : 0, (int)wl);
+  // WL copies only for W^T within LPF_WL_MAX (K <= 48 at N = 6K): instantiated for KS <= 2
+#define CLARUS_LPF_CB(XDT, LNV, WSV, KSV)                                                                  \
+  do {                                                                                                     \
+    if (!WSV && wl && KSV <= 2) {                                                                          \
+      lpf_allow_lds(reinterpret_cast<const void*>(&lpf_kernel<XDT, LNV, WSV, 2, KSV, !WSV && KSV <= 2>));  \
+      hipLaunchKernelGGL((lpf_kernel<XDT, LNV, WSV, 2, KSV, !WSV && KSV <= 2>), g, dim3(256), wl_bytes, s, \
+                         p);                                                                               \
+    } else {                                                                                               \
+      hipLaunchKernelGGL((lpf_kernel<XDT, LNV, WSV, 2, KSV, false>), g, dim3(256), 0, s, p);               \
+    }                                                                                                      \
+  } while (0)
+#define CLARUS_LPF_KS(XDT, LNV, WSV)                   \
+  do {                                                 \
+    switch (ks) {                                      \
+      case 2: CLARUS_LPF_CB(XDT, LNV, WSV, 2); break;  \
+      case 3: CLARUS_LPF_CB(XDT, LNV, WSV, 3); break;  \
+      case 4: CLARUS_LPF_CB(XDT, LNV, WSV, 4); break;  \
+      case 6: CLARUS_LPF_CB(XDT, LNV, WSV, 6); break;  \
+      default: CLARUS_LPF_CB(XDT, LNV, WSV, 8); break; \
+    }                                                  \
   } while (0)
   if (ln == 0) {
     if (x_dtype == DT_BF16) {
@@ -768,4 +888,52 @@ extern "C" int clarus_hip_linear_patch_filter(const void* x, int32_t x_dtype, co
 #undef CLARUS_LPF_KS
 #undef CLARUS_LPF_CB
   return check_launch("linear_patch_filter");
+}
+
+}  // namespace clarus
+
+using namespace clarus;
+
+extern "C" int clarus_hip_patch_filter(const void* x, int32_t x_dtype, int64_t ldx, const float* fwd,
+                                       const float* inv, const float* gain, const void* res, int32_t r_dtype,
+                                       void* out, int32_t o_dtype, int64_t batch, int64_t h, int64_t w, int64_t c,
+                                       void* stream) {
+  return run_patch_filter(false, x, x_dtype, ldx, fwd, inv, gain, res, r_dtype, out, o_dtype, batch, h, w, c, stream);
+}
+
+extern "C" int clarus_hip_patch_filter_rfft2(const void* x, int32_t x_dtype, int64_t ldx, const float* fwd,
+                                             const float* inv, const float* gain, const void* res, int32_t r_dtype,
+                                             void* out, int32_t o_dtype, int64_t batch, int64_t h, int64_t w,
+                                             int64_t c, void* stream) {
+  return run_patch_filter(true, x, x_dtype, ldx, fwd, inv, gain, res, r_dtype, out, o_dtype, batch, h, w, c, stream);
+}
+
+extern "C" int clarus_hip_patch_corr(const void* x, int32_t x_dtype, int64_t sn, int64_t sh, int64_t sw,
+                                     const float* fwd, const float* inv, float* out, int64_t batch, int64_t h,
+                                     int64_t w, int64_t c, void* stream) {
+  return run_patch_corr(false, x, x_dtype, sn, sh, sw, fwd, inv, out, batch, h, w, c, stream);
+}
+
+extern "C" int clarus_hip_patch_corr_rfft2(const void* x, int32_t x_dtype, int64_t sn, int64_t sh, int64_t sw,
+                                           const float* fwd, const float* inv, float* out, int64_t batch, int64_t h,
+                                           int64_t w, int64_t c, void* stream) {
+  return run_patch_corr(true, x, x_dtype, sn, sh, sw, fwd, inv, out, batch, h, w, c, stream);
+}
+
+extern "C" int clarus_hip_linear_patch_filter(const void* x, int32_t x_dtype, const void* wt, int32_t w_dtype,
+                                              const float* bias, int32_t ln, float ln_eps, const float* fwd,
+                                              const float* inv, const float* gain, const void* res, int32_t r_dtype,
+                                              void* out, int32_t o_dtype, int64_t batch, int64_t h, int64_t w,
+                                              int64_t k, int64_t n, void* stream) {
+  return run_linear_patch_filter(false, x, x_dtype, wt, w_dtype, bias, ln, ln_eps, fwd, inv, gain, res, r_dtype, out,
+                                 o_dtype, batch, h, w, k, n, stream);
+}
+
+extern "C" int clarus_hip_linear_patch_filter_rfft2(const void* x, int32_t x_dtype, const void* wt, int32_t w_dtype,
+                                                    const float* bias, int32_t ln, float ln_eps, const float* fwd,
+                                                    const float* inv, const float* gain, const void* res,
+                                                    int32_t r_dtype, void* out, int32_t o_dtype, int64_t batch,
+                                                    int64_t h, int64_t w, int64_t k, int64_t n, void* stream) {
+  return run_linear_patch_filter(true, x, x_dtype, wt, w_dtype, bias, ln, ln_eps, fwd, inv, gain, res, r_dtype, out,
+                                 o_dtype, batch, h, w, k, n, stream);
 }

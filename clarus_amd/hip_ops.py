@@ -879,7 +879,7 @@ class HipOps(Backend):
         gain = self.cached(f, "gain", lambda t: t.float().reshape(t.shape[0], -1).repeat_interleave(2, dim=1)
                            .contiguous())
         out = torch.empty((n, h, wd, c), device=x.device, dtype=odt)
-        _lib.check(self.lib.clarus_hip_patch_filter(
+        _lib.check(self.lib.clarus_hip_patch_filter_rfft2(
             x.data_ptr(), _lib.dtype_code(x.dtype), x.stride(2), fwd.data_ptr(), inv.data_ptr(), gain.data_ptr(),
             _lib.ptr(residual), _lib.dtype_code(residual.dtype) if residual is not None else 0, out.data_ptr(),
             _lib.dtype_code(odt), n, h, wd, c, self._stream(x)), "patch_filter")
@@ -887,7 +887,7 @@ class HipOps(Backend):
 
     def linear_patch_filter(self, x, w, bias, f, ln=False, ln_eps=1e-6, residual=None):
         """patch_filter(linear(x, w, bias, ln) kept fp32, f, residual) in one kernel
-        (clarus_hip_linear_patch_filter): the GEMM output goes from the MFMA accumulators
+        (clarus_hip_linear_patch_filter_rfft2): the GEMM output goes from the MFMA accumulators
         straight into the patch DFT, never to memory. Prologue arithmetic as linear's: LayerNorm /
         RMS inside the kernel in fp32 for K < split_min_k (or fp32 weights, K <= 256), else the
         rows pass rounded once to bf16 first (the reference's ln_rows for K > 128,
@@ -922,7 +922,7 @@ class HipOps(Backend):
         gain = self.cached(f, "gain", lambda t: t.float().reshape(t.shape[0], -1).repeat_interleave(2, dim=1)
                            .contiguous())
         out = torch.empty((n, h, wd, nout), device=x.device, dtype=self.dtype)
-        _lib.check(self.lib.clarus_hip_linear_patch_filter(
+        _lib.check(self.lib.clarus_hip_linear_patch_filter_rfft2(
             a.data_ptr(), _lib.dtype_code(a.dtype), wt.data_ptr(), _lib.dtype_code(wt.dtype), self._bias(bias).data_ptr(),
             code, float(ln_eps), fwd.data_ptr(), inv.data_ptr(), gain.data_ptr(), _lib.ptr(residual),
             _lib.dtype_code(residual.dtype) if residual is not None else 0, out.data_ptr(), _lib.dtype_code(self.dtype),
@@ -935,9 +935,9 @@ class HipOps(Backend):
             raise Unsupported("patch_corr: 8x8 patches, H and W multiples of 8, unit channel stride, >= 2c channels")
         fwd, inv = self._mats(x.device)
         out = torch.empty((n, h, w, c), device=x.device, dtype=torch.float32)
-        _lib.check(self.lib.clarus_hip_patch_corr(x.data_ptr(), _lib.dtype_code(x.dtype), x.stride(0), x.stride(1),
-                                                  x.stride(2), fwd.data_ptr(), inv.data_ptr(), out.data_ptr(), n, h,
-                                                  w, c, self._stream(x)), "patch_corr")
+        _lib.check(self.lib.clarus_hip_patch_corr_rfft2(
+            x.data_ptr(), _lib.dtype_code(x.dtype), x.stride(0), x.stride(1), x.stride(2), fwd.data_ptr(), inv.data_ptr(),
+            out.data_ptr(), n, h, w, c, self._stream(x)), "patch_corr")
         return out
 
     def ln_mul_linear(self, x, ln_w, ln_b, m, w, bias=None, m_act=None, residual=None, ln_eps=1e-5,

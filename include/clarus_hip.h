@@ -337,12 +337,11 @@ int clarus_hip_channel_attention_noalloc(const void* qkv, int32_t qkv_dtype, con
                                          int64_t heads, void* stream);
 
 /*
- * Per 8x8 patch and channel: y = irfft2(rfft2(patch) * g[c]) (+ residual), as fp32 FFTs in
- * registers, which need the gains only, where x and out lie within 2^29 elements; past them as the
- * dense real products  y = Inv[64 x 80] . (g_c * (Fwd[80 x 64] . x))  with
- * fwd [80][64] and inv [64][80] fp32, the matrices of rfft2 and irfft2 (clarus_amd/dft.py);
- * gain [c][80] fp32 (the filter per coefficient). x [batch, h, w, c] NHWC with pixel
- * stride ldx; h, w multiples of 8 (the caller reflect-pads other sizes).
+ * Per 8x8 patch and channel: y = Inv[64 x 80] . (g_c * (Fwd[80 x 64] . x)) (+ residual), dense real
+ * products with the caller's matrices; with those of rfft2 and irfft2 (clarus_amd/dft.py) this is
+ * irfft2(rfft2(patch) * g[c]). fwd [80][64] and inv [64][80] fp32; gain [c][80] fp32 (the filter per
+ * coefficient). x [batch, h, w, c] NHWC with pixel stride ldx; sizes that are no multiple of 8 are
+ * reflect-padded (h, w larger than the pad).
  * out [batch, h, w, c] contiguous, dtype o_dtype; residual contiguous like out or NULL.
  * replaces ops/torch_ref.py:253-270 patch_filter (torch-only in the reference)
  */
@@ -350,6 +349,16 @@ int clarus_hip_patch_filter(const void* x, int32_t x_dtype, int64_t ldx, const f
                             const float* inv, const float* gain, const void* res,
                             int32_t r_dtype, void* out, int32_t o_dtype, int64_t batch,
                             int64_t h, int64_t w, int64_t c, void* stream);
+
+/*
+ * The same with the transforms fixed as rfft2 and irfft2: fp32 FFTs in registers, which need the gains
+ * only, where x and out lie within 2^29 elements. fwd and inv have to be the matrices of rfft2 and
+ * irfft2; they are read past those sizes, where the dense products run.
+ */
+int clarus_hip_patch_filter_rfft2(const void* x, int32_t x_dtype, int64_t ldx, const float* fwd,
+                                  const float* inv, const float* gain, const void* res,
+                                  int32_t r_dtype, void* out, int32_t o_dtype, int64_t batch,
+                                  int64_t h, int64_t w, int64_t c, void* stream);
 
 /*
  * patch_filter(prologue(x) . W + bias) (+ residual) in one kernel: per 8x8 patch and output
@@ -362,9 +371,8 @@ int clarus_hip_patch_filter(const void* x, int32_t x_dtype, int64_t ldx, const f
  * (h, w >= 9), which for a per-pixel GEMM is the GEMM of the reflected pixels. out [batch, h, w, n]
  * contiguous (o_dtype); residual contiguous like out or NULL. k % 8 == 0. With bf16 weights the
  * GEMM's A values enter bf16 MFMAs as hi + lo pairs where they are not bf16 already (2^-16
- * relative per operand); with fp32 weights it runs on fp32 MFMAs. With bf16 x and weights and k <= 96
- * (192 without a prologue) the transforms run as fp32 FFTs, which need the gains only (fwd and inv being
- * the matrices of rfft2 and irfft2); otherwise as the DFT products of clarus_hip_patch_filter.
+ * relative per operand); with fp32 weights it runs on fp32 MFMAs. The DFT products are those of
+ * clarus_hip_patch_filter.
  * replaces kernels/freq.py:189-273 ln_gemm_patch_filter (ops/triton_cuda.py:260-272)
  */
 int clarus_hip_linear_patch_filter(const void* x, int32_t x_dtype, const void* wt, int32_t w_dtype,
@@ -374,15 +382,30 @@ int clarus_hip_linear_patch_filter(const void* x, int32_t x_dtype, const void* w
                                    int64_t k, int64_t n, void* stream);
 
 /*
+ * The same with the transforms fixed as rfft2 and irfft2 (fwd and inv have to be their matrices): with
+ * bf16 x and weights and k <= 96 (192 without a prologue) as fp32 FFTs, which need the gains only;
+ * otherwise as the dense products.
+ */
+int clarus_hip_linear_patch_filter_rfft2(const void* x, int32_t x_dtype, const void* wt, int32_t w_dtype,
+                                         const float* bias, int32_t ln, float ln_eps, const float* fwd,
+                                         const float* inv, const float* gain, const void* res,
+                                         int32_t r_dtype, void* out, int32_t o_dtype, int64_t batch,
+                                         int64_t h, int64_t w, int64_t k, int64_t n, void* stream);
+
+/*
  * FFTformer FSAS correlation (ops/torch_ref.py:278-288): per 8x8 patch,
  * irfft2(rfft2(q) * rfft2(k)) with q = x[..., :c], k = x[..., c:2c]; x has unit channel
  * stride and arbitrary batch / row / pixel strides (elements); out fp32 [batch, h, w, c].
- * fwd [80][64], inv [64][80] and the two forms as above.
+ * fwd [80][64] and inv [64][80] as for clarus_hip_patch_filter, a complex product per pair of
+ * coefficients; clarus_hip_patch_corr_rfft2 as clarus_hip_patch_filter_rfft2.
  * replaces kernels/freq.py:165-186 patch_corr
  */
 int clarus_hip_patch_corr(const void* x, int32_t x_dtype, int64_t sn, int64_t sh, int64_t sw,
                           const float* fwd, const float* inv, float* out, int64_t batch,
                           int64_t h, int64_t w, int64_t c, void* stream);
+int clarus_hip_patch_corr_rfft2(const void* x, int32_t x_dtype, int64_t sn, int64_t sh, int64_t sw,
+                                const float* fwd, const float* inv, float* out, int64_t batch,
+                                int64_t h, int64_t w, int64_t c, void* stream);
 
 /*
  * Depthwise 3x3 convolution, 'same' zero padding, dilation dil, fused gate (NHWC):

@@ -399,3 +399,101 @@ def test_fft_patch_corr(n, h, w, c, dt, hip_bf16, hip_f32):
     dense = hip.patch_corr(one, c)
     assert _lib.last_kernel().startswith("patch_kernel corr=1"), _lib.last_kernel()
     assert_fp32(dense.cpu(), ref[:1], rel=1e-5, what=f"dense patch_corr {h}x{w}x{c}")
+
+
+# ------------------------------------------------------------------ the C entries with the caller's matrices
+def _patches(t):
+    """[n, h, w, c] (sizes reflect-padded to multiples of 8) -> [n, ph, pw, c, 64] in fp64."""
+    n, h, w, c = t.shape
+    t = torch.nn.functional.pad(t.double().permute(0, 3, 1, 2), (0, -w % 8, 0, -h % 8), mode="reflect")
+    ph, pw = t.shape[2] // 8, t.shape[3] // 8
+    return t.view(n, c, ph, 8, pw, 8).permute(0, 2, 4, 1, 3, 5).reshape(n, ph, pw, c, 64)
+
+
+def _unpatch(y, h, w):
+    n, ph, pw, c, _ = y.shape
+    return y.view(n, ph, pw, c, 8, 8).permute(0, 1, 4, 2, 5, 3).reshape(n, ph * 8, pw * 8, c)[:, :h, :w]
+
+
+def _matrices(seed):
+    g = gen(seed)
+    return rnd(g, 80, 64, scale=1 / 8), rnd(g, 64, 80, scale=1 / 9)
+
+
+def assert_split(got, ref, mag, what):
+    """mag: the reference's formula on absolute values. A product of hi + lo operands is off by at most 3 * 2^-18 of
+    its magnitude (2^-18 for each operand, the dropped lo lo term), sums of up to 192 terms in fp32 by 192 * 2^-24 =
+    3 * 2^-18; at most four such products depend on each other or add up (corr: two forward, one inverse; linear: GEMM,
+    forward, inverse), with their sums 4 * (3 + 3) = 24."""
+    assert torch.isfinite(got).all(), what
+    worst = ((got.double() - ref).abs() / (mag * 24 * 2.0 ** -18)).max().item()
+    assert worst <= 1, f"{what}: {worst:.2f} of the bound"
+
+
+@pytest.mark.parametrize("n,h,w,c,dt,res", [(1, 13, 21, 33, torch.bfloat16, torch.float32), (2, 24, 40, 48, torch.float32, None),
+                                            (1, 64, 72, 96, torch.bfloat16, None), (1, 9, 16, 8, torch.float32, torch.bfloat16)])
+def test_patch_filter_callers_matrices(n, h, w, c, dt, res, gpu_device):
+    """clarus_hip_patch_filter computes Inv . (g_c * (Fwd . x)) with the matrices it is given, here random ones,
+    and gains that differ between a bin's two parts: patch_kernel, reflected edges and residuals."""
+    from clarus_amd import _lib
+    lib, g = _lib.load(), gen(h * w + c)
+    (fwd, inv), x, gain = _matrices(c), rnd(g, n, h, w, c, dtype=dt), rnd(g, c, 80)
+    r = None if res is None else rnd(g, n, h, w, c, dtype=res)
+    xd, fd, vd, gd, rd = (None if t is None else t.cuda() for t in (x, fwd, inv, gain, r))
+    out = torch.empty(n, h, w, c, device="cuda")
+    _lib.check(lib.clarus_hip_patch_filter(
+        xd.data_ptr(), _lib.dtype_code(dt), c, fd.data_ptr(), vd.data_ptr(), gd.data_ptr(), _lib.ptr(rd),
+        _lib.dtype_code(res) if res else 0, out.data_ptr(), _lib.F32, n, h, w, c, torch.cuda.current_stream().cuda_stream),
+        "patch_filter")
+    def formula(x, fwd, gain, inv, r):
+        return _unpatch((_patches(x) @ fwd.double().t() * gain.double()) @ inv.double().t(), h, w) + (0 if r is None else r)
+    ops = (x, fwd, gain, inv, None if r is None else r.double())
+    assert_split(out.cpu(), formula(*ops), formula(*(None if t is None else t.abs() for t in ops)), f"patch_filter {n}x{h}x{w}x{c}")
+    assert _lib.last_kernel().startswith("patch_kernel corr=0"), _lib.last_kernel()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_patch_corr_callers_matrices(dt, gpu_device):
+    """clarus_hip_patch_corr: Inv . (Fwd q * Fwd k), a complex product per pair, with random matrices."""
+    from clarus_amd import _lib
+    lib, g = _lib.load(), gen(11)
+    n, h, w, c = 2, 16, 24, 40
+    (fwd, inv), x = _matrices(5), rnd(g, n, h, w, 3 * c, dtype=dt)
+    xd, fd, vd = x.cuda(), fwd.cuda(), inv.cuda()
+    out = torch.empty(n, h, w, c, device="cuda")
+    _lib.check(lib.clarus_hip_patch_corr(xd.data_ptr(), _lib.dtype_code(dt), *xd.stride()[:3], fd.data_ptr(), vd.data_ptr(),
+                                         out.data_ptr(), n, h, w, c, torch.cuda.current_stream().cuda_stream), "patch_corr")
+    def formula(x, fwd, inv, minus):
+        q, k = ((_patches(x[..., s:s + c]) @ fwd.double().t()).unflatten(-1, (40, 2)) for s in (0, c))
+        re, im = q[..., 0] * k[..., 0] + minus * q[..., 1] * k[..., 1], q[..., 0] * k[..., 1] + q[..., 1] * k[..., 0]
+        return _unpatch(torch.stack((re, im), -1).flatten(-2) @ inv.double().t(), h, w)
+    assert_split(out.cpu(), formula(x, fwd, inv, -1), formula(x.abs(), fwd.abs(), inv.abs(), 1), "patch_corr")
+    assert _lib.last_kernel().startswith("patch_kernel corr=1"), _lib.last_kernel()
+
+
+@pytest.mark.parametrize("h,w,k,n,ln,dt", [(17, 40, 48, 96, 1, torch.bfloat16), (24, 31, 96, 288, 2, torch.bfloat16),
+                                           (45, 61, 64, 40, 0, torch.bfloat16), (16, 24, 144, 48, 0, torch.float32)])
+def test_linear_patch_filter_callers_matrices(h, w, k, n, ln, dt, gpu_device):
+    """clarus_hip_linear_patch_filter with random matrices, in the forms that its _rfft2 entry computes by FFTs and
+    one that it does not: W^T from LDS and from memory, whole patches per wave, reflected edges, a residual."""
+    from clarus_amd import _lib
+    lib, g = _lib.load(), gen(h + k)
+    (fwd, inv), x, gain = _matrices(n), rnd(g, 1, h, w, k, dtype=dt), rnd(g, n, 80)
+    wl, b, r = rnd(g, n, k, scale=k ** -0.5, dtype=dt), rnd(g, n, scale=0.1), rnd(g, 1, h, w, n, dtype=dt)
+    xd, wd, bd, fd, vd, gd, rd = (t.cuda() for t in (x, wl, b, fwd, inv, gain, r))
+    out = torch.empty(1, h, w, n, device="cuda")
+    code = _lib.dtype_code(dt)
+    _lib.check(lib.clarus_hip_linear_patch_filter(
+        xd.data_ptr(), code, wd.data_ptr(), code, bd.data_ptr(), ln, 1e-5, fd.data_ptr(), vd.data_ptr(), gd.data_ptr(),
+        rd.data_ptr(), code, out.data_ptr(), _lib.F32, 1, h, w, k, n, torch.cuda.current_stream().cuda_stream),
+        "linear_patch_filter")
+    rows = x.double()
+    if ln:
+        rows = rows - (rows.mean(-1, keepdim=True) if ln == 1 else 0)
+        rows = rows / (rows.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+    def formula(rows, wl, b, fwd, gain, inv, r):
+        z = rows @ wl.double().t() + b.double()
+        return _unpatch((_patches(z) @ fwd.double().t() * gain.double()) @ inv.double().t(), h, w) + r.double()
+    ops = (rows, wl, b, fwd, gain, inv, r)
+    assert_split(out.cpu(), formula(*ops), formula(*(t.abs() for t in ops)), f"linear_patch_filter {h}x{w} k{k} n{n}")
+    assert _lib.last_kernel().startswith("lpf_kernel"), _lib.last_kernel()
