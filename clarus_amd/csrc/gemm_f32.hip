@@ -4,19 +4,16 @@
 //
 // Restormer's deep levels in fp32 (K = 192 .. 1024). Bound: the fp32 MFMA rate. The general tiled kernel reads
 // A from global memory into each lane once per 64 channels and waits for it; here A and W^T pass through LDS.
-//   * Tile: TM pixels x 128 channels, 4 waves of TM / 2 x 64 on 32x32x2 MFMAs with W^T as the A operand (rows
+//   * Tile: 64 pixels x 128 channels, 4 waves of 32 x 64 on 32x32x2 MFMAs with W^T as the A operand (rows
 //     permuted so that a lane ends with 16 consecutive channels of a pixel).
 //   * K in chunks of 32: rows of 128 bytes copied global -> LDS directly, two buffers, the next chunk in flight
 //     during the current one's products. 16-byte units are XOR-swizzled with the row, so the 32 rows of a
 //     fragment read fall on distinct banks. Which k a lane half supplies is free as long as both operands
 //     agree: half h takes units 2 j + h, one 16-byte read feeding four MFMAs.
 //   * Row statistics come from the separate pass; a fragment is normalised as it is read.
-//   * TM = 64 or 128, whichever leaves less of the last round of tiles empty; tiles dealt in contiguous runs
-//     per XCD, the channel tiles of a pixel tile next to each other.
+//   * Tiles dealt in contiguous runs per XCD, the channel tiles of a pixel tile next to each other.
 // Measured (us, before -> now): 14400 rows, LayerNorm, 384 -> 1152 191 -> 146, 384 -> 2048 330 -> 241 (94 TFLOP/s of
 // 150 that a large fp32 product reaches on this card); + residual, 1024 -> 384 158 -> 116, 384 -> 384 68 -> 52.
-#include <algorithm>
-
 #include "capi.hpp"
 #include "gemm_f32_dispatch.hpp"
 #include "gemm_kernel.hpp"
@@ -25,13 +22,12 @@ namespace clarus {
 namespace {
 
 typedef __attribute__((ext_vector_type(16))) float f32x16;
-constexpr int F3_KC = 32, F3_TN = 128;
+constexpr int F3_KC = 32, F3_TN = 128, F3_TM = 64;
 __device__ __attribute__((aligned(256))) unsigned char g_f32_zero[256];
 
-template <int TM, bool STATS>
+template <bool STATS>
 __global__ void __launch_bounds__(256, 2) gemm_f32_kernel(const GemmP p, const int ntiles, const int tiles) {
-  constexpr int PT = TM / 64;                        // 32-pixel MFMA tiles per wave
-  constexpr int ROWS = F3_TN + TM;                   // W^T rows, then A rows
+  constexpr int ROWS = F3_TN + F3_TM;                // W^T rows, then A rows
   constexpr int COPIES = ROWS * 8 / 256;             // 16-byte units per lane and chunk
   constexpr int BUF = ROWS * 128;
   __shared__ __attribute__((aligned(16))) unsigned char lds[2][BUF];
@@ -40,7 +36,7 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_kernel(const GemmP p, const i
   const int per = (tiles + 7) / 8, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
   const int t = xcd * per + idx;
   if (idx >= per || t >= tiles) return;
-  const int64_t q0 = (int64_t)(t / ntiles) * TM;
+  const int64_t q0 = (int64_t)(t / ntiles) * F3_TM;
   const int n0 = (t % ntiles) * F3_TN;
   const int N = (int)p.n, K = (int)p.k;
   const int64_t bz = blockIdx.z;
@@ -70,25 +66,19 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_kernel(const GemmP p, const i
                                        (__attribute__((address_space(3))) void*)(dst + (wave + 4 * j) * 1024), 16, 0, 0);
     }
   };
-  const int wc = (wave & 1) * 64, wp = (wave >> 1) * (TM / 2);  // the wave's channels and pixels in the tile
-  float mean[PT], rstd[PT];
-#pragma unroll
-  for (int b = 0; b < PT; ++b) {
-    mean[b] = 0.f;
-    rstd[b] = 1.f;
-    if constexpr (STATS) {
-      const f32x2 st = *reinterpret_cast<const f32x2*>(p.stats + 2 * min(q0 + wp + 32 * b + lp, p.m - 1));
-      mean[b] = st[0];
-      rstd[b] = st[1];
-    }
+  const int wc = (wave & 1) * 64, wp = (wave >> 1) * (F3_TM / 2);  // the wave's channels and pixels in the tile
+  const int64_t q = q0 + wp + lp;  // the lane's pixel
+  float mean = 0.f, rstd = 1.f;
+  if constexpr (STATS) {
+    const f32x2 st = *reinterpret_cast<const f32x2*>(p.stats + 2 * min(q, p.m - 1));
+    mean = st[0];
+    rstd = st[1];
   }
-  f32x16 acc[2][PT];
+  f32x16 acc[2];
 #pragma unroll
   for (int c = 0; c < 2; ++c)
 #pragma unroll
-    for (int b = 0; b < PT; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[c][b][i] = 0.f;
+    for (int i = 0; i < 16; ++i) acc[c][i] = 0.f;
 
   const int nc = (K + F3_KC - 1) / F3_KC;
   wait_vmcnt<0>();  // the statistics: from here on only copies are counted
@@ -105,82 +95,64 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_kernel(const GemmP p, const i
 #pragma unroll
     for (int j = 0; j < F3_KC / 8; ++j) {
       const int place = ((2 * j + lh) ^ (lp & 7)) * 16;
-      f32x4 w[2], a[PT];
+      f32x4 w[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) w[i] = *reinterpret_cast<const f32x4*>(cur + (wc + 32 * i + lp) * 128 + place);
+      f32x4 a = *reinterpret_cast<const f32x4*>(cur + (F3_TN + wp + lp) * 128 + place);
+      if constexpr (STATS) {
 #pragma unroll
-      for (int b = 0; b < PT; ++b) {
-        a[b] = *reinterpret_cast<const f32x4*>(cur + (F3_TN + wp + 32 * b + lp) * 128 + place);
-        if constexpr (STATS) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a[b][e] = (a[b][e] - mean[b]) * rstd[b];
-        }
+        for (int e = 0; e < 4; ++e) a[e] = (a[e] - mean) * rstd;
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int b = 0; b < PT; ++b) acc[i][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[i][e], a[b][e], acc[i][b], 0, 0, 0);
+        for (int i = 0; i < 2; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[i][e], a[e], acc[i], 0, 0, 0);
     }
     barrier_keep_vm();  // every wave is done with this buffer before the copies two chunks on
   }
-  // ---- epilogue: pixel wp + 32 b + lp, channels c0 .. c0 + 15
+  // ---- epilogue: channels c0 .. c0 + 15 of the lane's pixel
+  if (q >= p.m) return;
 #pragma unroll
-  for (int b = 0; b < PT; ++b) {
-    const int64_t q = q0 + wp + 32 * b + lp;
-    if (q >= p.m) continue;
+  for (int i = 0; i < 2; ++i) {
+    const int c0 = n0 + wc + 32 * i + 16 * lh;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int c0 = n0 + wc + 32 * i + 16 * lh;
+    for (int j = 0; j < 2; ++j) {  // two runs of 8 channels (N is a multiple of 8)
+      const int c = c0 + 8 * j;
+      if (c >= N) continue;
+      float v[8];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {  // two runs of 8 channels (N is a multiple of 8)
-        const int c = c0 + 8 * j;
-        if (c >= N) continue;
-        float v[8];
+      for (int e = 0; e < 8; ++e) v[e] = acc[i][8 * j + e];
+      if (p.bias) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = acc[i][b][8 * j + e];
-        if (p.bias) {
+        for (int e = 0; e < 8; ++e) v[e] += p.bias[c + e];
+      }
+      if (p.act == ACT_GELU) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] += p.bias[c + e];
-        }
-        if (p.act == ACT_GELU) {
+        for (int e = 0; e < 8; ++e) v[e] = gelu_erf(v[e]);
+      }
+      if (p.scale) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = gelu_erf(v[e]);
-        }
-        if (p.scale) {
+        for (int e = 0; e < 8; ++e) v[e] *= p.scale[c + e] * p.out_scale;
+      } else if (p.out_scale != 1.0f) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] *= p.scale[c + e] * p.out_scale;
-        } else if (p.out_scale != 1.0f) {
+        for (int e = 0; e < 8; ++e) v[e] *= p.out_scale;
+      }
+      if (p.has_res) {
+        const int64_t ro = bz * p.r_bs + q * p.ldr + c;
+        const f32x8 r = p.r_dt == DT_BF16 ? load8<DT_BF16>((const unsigned short*)p.res + ro) : load8<DT_F32>((const float*)p.res + ro);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] *= p.out_scale;
-        }
-        if (p.has_res) {
-          const int64_t ro = bz * p.r_bs + q * p.ldr + c;
-          const f32x8 r = p.r_dt == DT_BF16 ? load8<DT_BF16>((const unsigned short*)p.res + ro) : load8<DT_F32>((const float*)p.res + ro);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] += r.v[e];
-        }
-        const int64_t co = bz * p.c_bs + q * p.ldc + c;
-        if (p.c_dt == DT_BF16) {
-          *reinterpret_cast<u32x4*>((unsigned short*)p.c + co) =
-              u32x4{pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]), pack2_bf16(v[4], v[5]), pack2_bf16(v[6], v[7])};
-        } else {
-          *reinterpret_cast<f32x4*>((float*)p.c + co) = f32x4{v[0], v[1], v[2], v[3]};
-          *reinterpret_cast<f32x4*>((float*)p.c + co + 4) = f32x4{v[4], v[5], v[6], v[7]};
-        }
+        for (int e = 0; e < 8; ++e) v[e] += r.v[e];
+      }
+      const int64_t co = bz * p.c_bs + q * p.ldc + c;
+      if (p.c_dt == DT_BF16) {
+        *reinterpret_cast<u32x4*>((unsigned short*)p.c + co) =
+            u32x4{pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]), pack2_bf16(v[4], v[5]), pack2_bf16(v[6], v[7])};
+      } else {
+        *reinterpret_cast<f32x4*>((float*)p.c + co) = f32x4{v[0], v[1], v[2], v[3]};
+        *reinterpret_cast<f32x4*>((float*)p.c + co + 4) = f32x4{v[4], v[5], v[6], v[7]};
       }
     }
   }
-}
-
-template <int TM>
-void launch_f32(const GemmP& p, int64_t batch, hipStream_t s) {
-  const int ntiles = (int)cdiv(p.n, F3_TN), tiles = (int)(cdiv(p.m, TM) * ntiles);
-  note_kernel("gemm_f32_kernel tm=%d stats=%d", TM, p.stats != nullptr);
-  const dim3 g((unsigned)(cdiv(tiles, 8) * 8), 1, (unsigned)batch);
-  if (p.stats) hipLaunchKernelGGL((gemm_f32_kernel<TM, true>), g, dim3(256), 0, s, p, ntiles, tiles);
-  else hipLaunchKernelGGL((gemm_f32_kernel<TM, false>), g, dim3(256), 0, s, p, ntiles, tiles);
 }
 
 }  // namespace
@@ -188,15 +160,16 @@ void launch_f32(const GemmP& p, int64_t batch, hipStream_t s) {
 bool gemm_f32_fits(const GemmP& p, int a_dt, int w_dt, int64_t batch) {
   return a_dt == DT_F32 && w_dt == DT_F32 && p.k > 128 && p.n % 8 == 0 && p.c_mode == CM_ROWS && p.vec_out == 2 &&
          (!p.has_res || p.vec_res == 2) && (p.act == ACT_NONE || p.act == ACT_GELU) && batch < 65536 &&
-         p.k < (1 << 28) && p.n < (1 << 24) && cdiv(p.m, 64) * cdiv(p.n, F3_TN) < ((int64_t)1 << 30) &&
+         p.k < (1 << 28) && p.n < (1 << 24) && cdiv(p.m, F3_TM) * cdiv(p.n, F3_TN) < ((int64_t)1 << 30) &&
          (p.pro == PRO_NONE || ((p.pro == PRO_LN || p.pro == PRO_RMS) && p.stats && batch == 1));
 }
 
 void launch_gemm_f32(const GemmP& p, int64_t batch, hipStream_t s) {
-  const int64_t nt = cdiv(p.n, F3_TN) * batch, cus = device_cus();
-  const int64_t c128 = cdiv(cdiv(p.m, 128) * nt, cus) * 2, c64 = cdiv(cdiv(p.m, 64) * nt, cus);
-  if (c64 <= c128) launch_f32<64>(p, batch, s);
-  else launch_f32<128>(p, batch, s);
+  const int ntiles = (int)cdiv(p.n, F3_TN), tiles = (int)(cdiv(p.m, F3_TM) * ntiles);
+  note_kernel("gemm_f32_kernel stats=%d", p.stats != nullptr);
+  const dim3 g((unsigned)(cdiv(tiles, 8) * 8), 1, (unsigned)batch);
+  if (p.stats) hipLaunchKernelGGL((gemm_f32_kernel<true>), g, dim3(256), 0, s, p, ntiles, tiles);
+  else hipLaunchKernelGGL((gemm_f32_kernel<false>), g, dim3(256), 0, s, p, ntiles, tiles);
 }
 
 }  // namespace clarus

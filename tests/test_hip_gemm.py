@@ -1798,8 +1798,7 @@ def test_smallm_kernel(m, k, n, kind, xdt, hip_bf16):
     (8200, 136, 40, "plain"), (4100, 200, 136, "ln"), (2049, 384, 520, "rms"), (8193, 160, 128, "res"), (3000, 264, 392, "gelu"),
     (16500, 136, 1160, "plain")])
 def test_gemm_f32_kernel(m, k, n, kind, hip_f32):
-    """linear in fp32 on gemm_f32_kernel (both tile heights): remainders of its pixel and channel tiles and of its
-    32-k chunks, statistics of the separate pass, residual and scale, GELU, against the oracle within 1e-5."""
+    """linear in fp32 on gemm_f32_kernel: remainders of its pixel and channel tiles and of its 32-k chunks, statistics of the separate pass, residual and scale, GELU, against the oracle within 1e-5."""
     from clarus_amd import _lib
     g = torch.Generator().manual_seed(m + k)
     x, w = torch.randn(1, 1, m, k, generator=g), torch.randn(k, n, generator=g) / k ** 0.5
