@@ -61,7 +61,10 @@ __global__ void __launch_bounds__(256, 2) gemm_f32_kernel(const GemmP p, const i
   auto issue = [&](int k0, unsigned char* dst) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < COPIES; ++j) {
-      const void* s = k0 + uk[j] < K ? (const void*)(src[j] + k0) : (const void*)g_f32_zero;
+      // past K W^T is zero and the operand must be finite: a normalised row repeats its last unit there, since
+      // (0 - mean) * rstd can overflow (rows of one large value)
+      const void* pad = STATS && j >= F3_TN / 32 ? (const void*)(src[j] - uk[j] + K - 4) : (const void*)g_f32_zero;
+      const void* s = k0 + uk[j] < K ? (const void*)(src[j] + k0) : pad;
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)s,
                                        (__attribute__((address_space(3))) void*)(dst + (wave + 4 * j) * 1024), 16, 0, 0);
     }

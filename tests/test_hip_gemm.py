@@ -1812,6 +1812,18 @@ def test_gemm_f32_kernel(m, k, n, kind, hip_f32):
     assert_fp32(got.cpu(), TorchRef(torch.float32, "cpu").linear(x, w, b, scale=sc, residual=res, **kw), what=f"f32 {m}x{k}x{n} {kind}")
 
 
+def test_gemm_f32_padding_of_constant_rows(hip_f32):
+    """K past its last 32-k chunk is no part of a row: rows of one large value have variance 0, so their LayerNorm is
+    exactly 0 and the output the bias, while (0 - mean) * rstd of a padding element would overflow."""
+    from clarus_amd import _lib
+    g = torch.Generator().manual_seed(8)
+    m, k, n = 4100, 200, 136
+    x, w, b = torch.full((1, 1, m, k), 2.0 ** 119), torch.randn(k, n, generator=g), torch.randn(n, generator=g)
+    got = hip_f32.linear(x.cuda(), w.cuda(), b.cuda(), ln=True)
+    assert _lib.last_kernel().startswith("gemm_f32_kernel"), _lib.last_kernel()
+    assert torch.equal(got.cpu(), b.expand(1, 1, m, n))
+
+
 def test_gemm_f32_per_image(hip_f32):
     """linear_per_image in fp32 on gemm_f32_kernel: two images, a channel slice of a wider tensor, a residual."""
     from clarus_amd import _lib
