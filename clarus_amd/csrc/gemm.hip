@@ -369,13 +369,12 @@ extern "C" int clarus_hip_gemm(const ClarusGemmArgs* a, void* stream) {
                      (hipStream_t)stream);
     p.stats = a->stats;
   }
-  // fp32 operands with K > 128: the LDS-tiled fp32 kernel (tile 21 forces it) from 128 tiles of 64 pixels x 128
-  // channels on; with fewer the 64 x 64 tiles below fill more of the GPU (us, general / LDS-tiled: 3000 rows
-  // 384 -> 384, 141 tiles 31.0 / 24.8; 1176 rows 192 -> 576, 95 tiles 18.0 / 21.2; 384 -> 384, 57 tiles 21.2 / 23.4)
+  // fp32 operands with K > 128: the LDS-tiled fp32 kernel (tile 21 forces it) where gemm_f32_faster says so
   {
     const bool f32_ok = a->a_mode == CLARUS_A_ROWS && !a->gate && gemm_f32_fits(p, a->a_dtype, a->w_dtype, a->batch);
     CLARUS_REQUIRE(a->tile != 21 || f32_ok, "gemm: the LDS-tiled fp32 kernel does not take this problem");
-    if (a->tile == 21 || (a->tile == 0 && f32_ok && cdiv(a->m, 64) * cdiv(a->n, 128) * a->batch >= 128)) {
+    if (a->tile == 21 ||
+        (a->tile == 0 && f32_ok && gemm_f32_faster(a->m, a->n, a->k, a->batch, a->pro != PRO_NONE, device_cus()))) {
       launch_gemm_f32(p, a->batch, (hipStream_t)stream);
       return check_launch("gemm");
     }

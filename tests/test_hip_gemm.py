@@ -1795,7 +1795,7 @@ def test_smallm_kernel(m, k, n, kind, xdt, hip_bf16):
 
 # ------------------------------------------------------------------ LDS-tiled fp32 kernel (K > 128)
 @pytest.mark.parametrize("m,k,n,kind", [
-    (8200, 136, 40, "plain"), (4100, 200, 136, "ln"), (2049, 384, 520, "rms"), (8193, 160, 128, "res"), (3000, 264, 392, "gelu"),
+    (8200, 136, 40, "plain"), (6000, 200, 136, "ln"), (2049, 384, 520, "rms"), (8193, 160, 128, "res"), (3000, 264, 392, "gelu"),
     (16500, 136, 1160, "plain")])
 def test_gemm_f32_kernel(m, k, n, kind, hip_f32):
     """linear in fp32 on gemm_f32_kernel: remainders of its pixel and channel tiles and of its 32-k chunks, statistics of the separate pass, residual and scale, GELU, against the oracle within 1e-5."""
@@ -1812,12 +1812,28 @@ def test_gemm_f32_kernel(m, k, n, kind, hip_f32):
     assert_fp32(got.cpu(), TorchRef(torch.float32, "cpu").linear(x, w, b, scale=sc, residual=res, **kw), what=f"f32 {m}x{k}x{n} {kind}")
 
 
+@pytest.mark.parametrize("m,k,n,ln,tiled", [
+    (5000, 136, 192, True, False), (5000, 136, 192, False, False), (6000, 136, 320, True, False),  # more rounds than 64 x 64 tiles'
+    (40000, 136, 48, False, False), (8192, 136, 96, True, False), (8192, 136, 96, False, True),    # half-empty channel tiles
+    (8192, 136, 128, False, False), (8192, 1024, 128, False, True), (3000, 384, 384, True, True),
+    (8192, 136, 24, True, True), (4000, 136, 24, False, False), (40000, 136, 24, False, False)])   # up to 32 channels
+def test_gemm_f32_routing(m, k, n, ln, tiled, hip_f32):
+    """fp32 linear past K = 128 runs on gemm_f32_kernel or on the general kernel, whichever takes fewer rounds of tiles
+    over the 256 CUs (and the two exceptions of that rule), with the same results."""
+    from clarus_amd import _lib
+    g = torch.Generator().manual_seed(m + n)
+    x, w, b = torch.randn(1, 1, m, k, generator=g), torch.randn(k, n, generator=g) / k ** 0.5, torch.randn(n, generator=g)
+    got = hip_f32.linear(x.cuda(), w.cuda(), b.cuda(), ln=ln)
+    assert _lib.last_kernel().startswith("gemm_f32_kernel" if tiled else "gemm_kernel"), _lib.last_kernel()
+    assert_fp32(got.cpu(), TorchRef(torch.float32, "cpu").linear(x, w, b, ln=ln), what=f"f32 routing {m}x{k}x{n}")
+
+
 def test_gemm_f32_padding_of_constant_rows(hip_f32):
     """K past its last 32-k chunk is no part of a row: rows of one large value have variance 0, so their LayerNorm is
     exactly 0 and the output the bias, while (0 - mean) * rstd of a padding element would overflow."""
     from clarus_amd import _lib
     g = torch.Generator().manual_seed(8)
-    m, k, n = 4100, 200, 136
+    m, k, n = 6000, 200, 136
     x, w, b = torch.full((1, 1, m, k), 2.0 ** 119), torch.randn(k, n, generator=g), torch.randn(n, generator=g)
     got = hip_f32.linear(x.cuda(), w.cuda(), b.cuda(), ln=True)
     assert _lib.last_kernel().startswith("gemm_f32_kernel"), _lib.last_kernel()
