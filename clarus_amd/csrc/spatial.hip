@@ -621,6 +621,20 @@ static int dw_tile_shape(int64_t units, int64_t n, int64_t H, int64_t W, bool ga
   return th;
 }
 
+// Dilation 1 on the per-pixel kernel all the same: more than 256 input channels (it splits those over workgroups) of
+// few pixels, where a launch is one chain of latencies and the tiled kernel's, copy, barrier and walk, is the longer.
+// fp32, whose tiles have one buffer: up to 4096 pixels and 2^21 outputs, with a gate 3000 and 1.25 million (us, per
+// pixel / tiled: 45 x 61, 288 channels 5.7 / 6.6, gate 384 -> 192 5.5 / 6.7; 24 x 49, GELU gate 2048 -> 1024 8.1 / 10.1; past
+// the lines 64 x 64, 576 channels 9.9 / 8.6, 45 x 61 gate 1152 -> 576 12.0 / 9.0). bf16 without a gate: 6-row tiles of
+// which only up to an eighth of the CUs get a second (45 x 61, 1152 channels 8.0 / 8.9; 64 x 64, 1024, three
+// eighths: 9.1 / 9.1).
+static bool dw_per_pixel(int64_t pixels, int64_t c, int64_t cout, bool gate, bool f32, int th, int64_t tiles) {
+  if (c <= 256) return false;
+  if (f32) return gate ? pixels <= 3000 && pixels * cout <= 1250000 : pixels <= 4096 && pixels * cout <= (1 << 21);
+  const int64_t cus = device_cus();
+  return !gate && th == 6 && pixels <= 6144 && tiles > cus && 8 * tiles <= 9 * cus;
+}
+
 extern "C" int clarus_hip_dwconv3x3(const void* x, int32_t x_dtype, const float* w, const float* bias, void* out,
                                     int32_t o_dtype, int64_t n, int64_t h, int64_t wd, int64_t c, int32_t dil,
                                     int32_t gate, int32_t act, void* stream) {
@@ -659,15 +673,13 @@ extern "C" int clarus_hip_dwconv3x3(const void* x, int32_t x_dtype, const float*
   } while (0)
   // LDS-tiled kernel: every call with dilation 1 whose tile rows fit 2^31-byte buffer ranges and whose
   // tile count fits 30 bits (it needs no alignment of taps and bias); the per-pixel kernel keeps dilated
-  // taps, whose halo would be larger than the tile, and images past those ranges. Down to 24 x 30 pixels
-  // the tiled form is the faster or even (us, before -> now: fp32 144 channels 10.6 -> 7.2, 288 channels at
-  // 24 x 49 6.9 -> 7.3, bf16 7.1 -> 6.7).
+  // taps, whose halo would be larger than the tile, images past those ranges, and what dw_per_pixel names.
   {
-    const int oes = o_dtype == DT_BF16 ? 2 : 4;
     DwTileP g{};
     const int th = dw_tile_shape(cdiv(cout, gate ? 4 : 8), n, h, wd, gate != 0, x_dtype == DT_F32, g);
     const int64_t ptiles = n * cdiv(h, th) * cdiv(wd, g.tw);
-    if (dil == 1 && (th + 2) * (wd + 2) * c * 4 < ((int64_t)1 << 31) && ptiles < ((int64_t)1 << 30)) {
+    if (dil == 1 && (th + 2) * (wd + 2) * c * 4 < ((int64_t)1 << 31) && ptiles < ((int64_t)1 << 30) &&
+        !dw_per_pixel(n * h * wd, c, cout, gate != 0, x_dtype == DT_F32, th, g.nslices * ptiles)) {
       g.tiles_y = (int)cdiv(h, th);
       g.tiles_x = (int)cdiv(wd, g.tw);
       g.ptiles = (int)ptiles;
@@ -709,6 +721,7 @@ extern "C" int clarus_hip_dwconv3x3(const void* x, int32_t x_dtype, const float*
       return check_launch("dwconv3x3");
     }
   }
+  note_kernel("dwconv3x3_kernel gate=%d dil=%d", gate, (int)dil);
   if (x_dtype == DT_BF16) {
     if (gate == 1) DW_LAUNCH(DT_BF16, 1); else if (gate == 2) DW_LAUNCH(DT_BF16, 2); else DW_LAUNCH(DT_BF16, 0);
   } else {

@@ -272,9 +272,26 @@ def test_dwconv_tile_forms(n, h, w, c, gate, act, dt, hip_bf16, hip_f32):
     off[1:] = b
     hip = hip_bf16 if dt == torch.bfloat16 else hip_f32
     got = hip.dwconv(x.cuda(), wt.cuda(), off.cuda()[1:], gate=gate, act=act)
-    assert _lib.last_kernel().startswith("dw_tile_kernel"), _lib.last_kernel()
+    kernel = "dwconv3x3_kernel" if dt == torch.float32 and c > 256 else "dw_tile_kernel"  # few pixels of many channels
+    assert _lib.last_kernel().startswith(kernel), _lib.last_kernel()
     check(got.cpu(), TorchRef(torch.float32, "cpu").dwconv(x, wt, b, gate=gate, act=act),
           f"dwconv tile {n}x{h}x{w}x{c} gate={gate} act={act} {dt}")
+
+
+@pytest.mark.parametrize("h,w,c,gate,dt,tiled", [
+    (64, 64, 512, False, "fp32", False), (64, 64, 520, False, "fp32", True), (45, 92, 288, False, "fp32", True),
+    (50, 60, 832, True, "fp32", False), (50, 60, 848, True, "fp32", True), (59, 51, 272, "gelu", "fp32", True),
+    (16, 16, 256, False, "fp32", True), (16, 16, 264, False, "fp32", False),
+    (45, 61, 1152, False, "bf16", False), (64, 64, 1024, False, "bf16", True), (45, 61, 1152, True, "bf16", True)])
+def test_dwconv_routing(h, w, c, gate, dt, tiled, hip_bf16, hip_f32):
+    """Both sides of every line between the tiled and the per-pixel kernel at dilation 1, against the oracle."""
+    from clarus_amd import _lib
+    g = gen(c + w)
+    x = rnd(g, 1, h, w, c, dtype=torch.float32 if dt == "fp32" else torch.bfloat16)
+    wt, b = rnd(g, c, 1, 3, 3, scale=0.3), rnd(g, c, scale=0.5)
+    got = (hip_f32 if dt == "fp32" else hip_bf16).dwconv(x.cuda(), wt.cuda(), b.cuda(), gate=gate)
+    assert _lib.last_kernel().startswith("dw_tile_kernel" if tiled else "dwconv3x3_kernel"), _lib.last_kernel()
+    check(got.cpu(), TorchRef(torch.float32, "cpu").dwconv(x, wt, b, gate=gate), f"dwconv routing {h}x{w}x{c} gate={gate} {dt}")
 
 
 def test_dwconv_bf16_in_fp32_out(hip_bf16):
