@@ -50,7 +50,9 @@ __global__ void __launch_bounds__(64 * LF_WAVES, 2) fft_lpf_kernel(const LpfFftP
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lp = lane & 31, lh = lane >> 5;
   const int H = p.h, W = p.w, K = p.k, N = p.n;
-  const int ph = (H + 7) / 8, pw = (W + 7) / 8, ctiles = (N + 31) / 32;
+  const int ph = (H + 7) / 8, pw = (W + 7) / 8;
+  const int ctall = (N + 31) / 32;  // the workgroup's channel tiles [ct0, ct0 + ctiles): all of them but for few patches
+  const int ct0 = ctall * blockIdx.y / gridDim.y, ctiles = ctall * (blockIdx.y + 1) / gridDim.y - ct0;
   const float invk = 1.0f / (float)K;
 
   auto patch_of = [&](int64_t pt, int64_t& n, int& py, int& px) __attribute__((always_inline)) {
@@ -145,7 +147,7 @@ __global__ void __launch_bounds__(64 * LF_WAVES, 2) fft_lpf_kernel(const LpfFftP
     while (i0 < i1) {
       // ---- one channel tile: weights, bias and gain factors of the lane's channel
       const int ct = i0 / PB, iend = min(i1, (ct + 1) * PB);
-      const int ch = ct * 32 + lp, chl = min(ch, N - 1);
+      const int ch = (ct0 + ct) * 32 + lp, chl = min(ch, N - 1);
       bf16x8 wv[KS];
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
@@ -287,16 +289,25 @@ __global__ void __launch_bounds__(64 * LF_WAVES, 2) fft_lpf_kernel(const LpfFftP
   }
 }
 
+template <int KS, bool PRO, int PB>
+void launch_pb(const LpfFftP& p, dim3 grid, hipStream_t s) {
+  note_kernel("fft_lpf_kernel pro=%d ks=%d pb=%d grid=%ux%u", (int)PRO, KS, PB, grid.x, grid.y);
+  hipLaunchKernelGGL((fft_lpf_kernel<KS, PRO, PB>), grid, dim3(64 * LF_WAVES), 0, s, p);
+}
+
 template <int KS, bool PRO>
 void launch_t(const LpfFftP& p, hipStream_t s) {
-  // one workgroup per CU with an even share of the patches, PB of them in LDS at a time (96 KiB); one patch per
-  // workgroup where that leaves CUs idle (45 x 61, 48 -> 288: 34 -> 13 us). Six waves with 72 KiB and two
-  // workgroups per CU: 342 us against 304 at 720 x 1280, 48 -> 288.
+  // one workgroup per CU (its registers fill it) with an even share of the patches, PB of them in LDS at a time
+  // (96 KiB). Up to as many patches as CUs: one per workgroup (45 x 61, 48 -> 288: 34 -> 13 us), and its channel tiles on
+  // several workgroups, up to one tile per wave, while CUs are left (16 x 16, 96 -> 576 without a prologue 16.7 -> 8.0 us).
+  // Between one and two patches per CU, batches of two, not two rounds of workgroups: 176 x 184, 192 -> 48 21.1 -> 10.8.
+  // Six waves with 72 KiB and two workgroups per CU: 342 us against 304 at 720 x 1280, 48 -> 288.
   constexpr int PB = KS * (PRO ? 2 : 1) <= 6 ? 8 : KS * (PRO ? 2 : 1) <= 8 ? 6 : 4;
-  if (p.patches < 2LL * device_cus())
-    hipLaunchKernelGGL((fft_lpf_kernel<KS, PRO, 1>), dim3((unsigned)p.patches), dim3(64 * LF_WAVES), 0, s, p);
-  else
-    hipLaunchKernelGGL((fft_lpf_kernel<KS, PRO, PB>), dim3((unsigned)device_cus()), dim3(64 * LF_WAVES), 0, s, p);
+  const int64_t cus = device_cus();
+  if (p.patches >= 2 * cus) return launch_pb<KS, PRO, PB>(p, dim3((unsigned)cus), s);
+  if (p.patches > cus) return launch_pb<KS, PRO, 2>(p, dim3((unsigned)cus), s);
+  const dim3 grid((unsigned)p.patches, (unsigned)std::min(cdiv(cdiv(p.n, 32), LF_WAVES), cus / p.patches));
+  launch_pb<KS, PRO, 1>(p, grid, s);
 }
 
 }  // namespace
@@ -304,7 +315,6 @@ void launch_t(const LpfFftP& p, hipStream_t s) {
 bool launch_lpf_fft(const LpfFftP& p, bool pro, hipStream_t s) {
   if (p.k % 8 || (int64_t)8 * p.w * p.n * 4 >= ((int64_t)1 << 29)) return false;
   const int ks = (p.k + 15) / 16;
-  note_kernel("fft_lpf_kernel pro=%d ks=%d", (int)pro, ks);
   if (pro) {
     if (ks <= 2) launch_t<2, true>(p, s);
     else if (ks == 3) launch_t<3, true>(p, s);

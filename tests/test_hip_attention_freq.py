@@ -278,7 +278,9 @@ def test_linear_patch_filter_fused_model_shapes(h, w, k, nout, ln, res, dt, hip_
     dv = [None if t is None else t.cuda() for t in (x, wl, b, f, rr)]
     print(f"[lpf] {dt} {h}x{w} k{k} n{nout} ln={ln} res={res}", flush=True)
     got = hip.linear_patch_filter(*dv[:4], ln=ln, ln_eps=1e-5, residual=dv[4])
-    assert "lpf_kernel" in _lib.last_kernel(), _lib.last_kernel()
+    # FFTs where the rows reach the kernel as bf16 with K <= 96 under a prologue or K <= 192 without one
+    fft = dt == torch.bfloat16 and k <= (96 if ln else 192)
+    assert _lib.last_kernel().startswith("fft_lpf_kernel" if fft else "lpf_kernel"), _lib.last_kernel()
     saved = HipOps.fuse_patch_filter
     try:
         HipOps.fuse_patch_filter = False
@@ -339,12 +341,22 @@ def test_patch_corr(dt, hip_bf16, hip_f32):
         assert_fp32(hip.patch_corr(fn(bd), c).cpu(), REF.patch_corr(fn(base), c), rel=1e-5, what=f"patch_corr {name}")
 
 
-@pytest.mark.parametrize("h,w,k,n,ln,res", [
-    (9, 9, 8, 8, False, False), (17, 40, 24, 40, True, False), (45, 61, 48, 288, True, True),
-    (24, 40, 96, 72, "rms", False), (33, 16, 192, 40, False, True), (200, 192, 48, 33, True, False),
-    (168, 200, 88, 40, True, False), (176, 184, 136, 24, False, False), (168, 200, 16, 8, "rms", True)])
-def test_fft_lpf_kernel(h, w, k, n, ln, res, hip_bf16):
-    """linear_patch_filter with FFT patch transforms: one patch per workgroup and several (over 512 patches),
+@pytest.mark.parametrize("h,w,k,n,ln,res,form", [
+    # up to as many patches as CUs: one per workgroup, its channel tiles on one workgroup or several
+    (9, 9, 8, 8, False, False, "ks=3 pb=1 grid=4x1"), (17, 40, 24, 40, True, False, "ks=2 pb=1 grid=15x1"),
+    (45, 61, 48, 288, True, True, "ks=3 pb=1 grid=48x2"), (24, 40, 96, 72, "rms", False, "ks=6 pb=1 grid=15x1"),
+    (33, 16, 192, 40, False, True, "ks=12 pb=1 grid=10x1"), (16, 24, 96, 570, False, False, "ks=6 pb=1 grid=6x3"),
+    (96, 104, 64, 296, True, True, "ks=4 pb=1 grid=156x1"), (16, 17, 128, 520, False, False, "ks=8 pb=1 grid=6x3"),
+    # up to two per CU: batches of two and of one
+    (176, 184, 136, 24, False, False, "ks=12 pb=2"), (136, 144, 64, 40, True, True, "ks=4 pb=2"),
+    (129, 136, 40, 72, False, False, "ks=3 pb=2"),
+    # more: a full batch of 8, 6 or 4 and a partial one, some with reflected columns
+    (376, 398, 48, 33, True, False, "ks=3 pb=8"), (376, 398, 16, 8, "rms", True, "ks=2 pb=8"),
+    (376, 398, 40, 48, False, False, "ks=3 pb=8"), (376, 398, 96, 24, False, True, "ks=6 pb=8"),
+    (376, 280, 64, 40, True, False, "ks=4 pb=6"), (376, 280, 128, 24, False, False, "ks=8 pb=6"),
+    (376, 280, 88, 40, True, False, "ks=6 pb=4"), (376, 280, 192, 24, False, True, "ks=12 pb=4")])
+def test_fft_lpf_kernel(h, w, k, n, ln, res, form, hip_bf16):
+    """linear_patch_filter with FFT patch transforms, every form on 256 CUs: one patch per workgroup, two and batches,
     partial batches, channel tiles and 16-k steps, reflected edges, against the oracle in fp32 on the same bf16
     operands (gains without the symmetry of a real filter's spectrum in columns 0 and 4)."""
     from clarus_amd import _lib
@@ -354,7 +366,7 @@ def test_fft_lpf_kernel(h, w, k, n, ln, res, hip_bf16):
     rr = rnd(g, 1, h, w, n).bfloat16() if res else None
     got = hip_bf16.linear_patch_filter(x.cuda(), wl.cuda(), b.cuda(), f.cuda(), ln=ln, ln_eps=1e-5,
                                        residual=None if rr is None else rr.cuda())
-    assert _lib.last_kernel().startswith("fft_lpf_kernel"), _lib.last_kernel()
+    assert _lib.last_kernel().startswith(f"fft_lpf_kernel pro={int(bool(ln))} {form}"), _lib.last_kernel()
     ref = REF.linear_patch_filter(x, wl, b, f, ln=ln, ln_eps=1e-5, residual=rr)
     assert_bf16(got.cpu(), ref, f"fft lpf {h}x{w} k{k} n{n}")
 
