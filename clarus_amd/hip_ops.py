@@ -224,7 +224,9 @@ class HipOps(Backend):
               ln_eps=1e-6, out_scale=1.0, tile=0, wp=None):
         h, w, oh, ow, pt, pl = geom
         stats = None
-        if (pro & 0xff) in (_lib.PRO_LN, _lib.PRO_RMS, _lib.PRO_LNMUL) and k > 128 and batch == 1 and wp is None:
+        # tile 20, the few-row kernel, computes them from its registers
+        if ((pro & 0xff) in (_lib.PRO_LN, _lib.PRO_RMS, _lib.PRO_LNMUL) and k > 128 and batch == 1 and wp is None
+                and tile != 20):
             stats = torch.empty(2 * m, device=a.device, dtype=torch.float32)  # row statistics scratch
         args = _lib.GemmArgs(
             a=a.data_ptr(), wt=wt.data_ptr(), c=c.data_ptr(), bias=_lib.ptr(bias), scale=_lib.ptr(scale),

@@ -1793,6 +1793,19 @@ def test_smallm_kernel(m, k, n, kind, xdt, hip_bf16):
     assert e <= tol, f"smallm {m}x{k}x{n} {kind}: {e:.2e}"
 
 
+def test_smallm_allocates_its_output_only(hip_bf16):
+    """A LayerNorm linear on the few-row kernel takes no statistics scratch: one allocation, the output."""
+    from clarus_amd import _lib
+    g = torch.Generator().manual_seed(5)
+    x, w, b = (t.cuda() for t in (torch.randn(1, 28, 48, 256, generator=g), torch.randn(256, 512, generator=g).bfloat16(),
+                                  torch.randn(512, generator=g)))
+    out = hip_bf16.linear(x, w, b, ln=True)  # the weight's layout is made once
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    again = hip_bf16.linear(x, w, b, ln=True)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == 1
+    assert _lib.last_kernel().startswith("gemm_smallm_kernel pro=1") and torch.equal(out, again)
+
+
 # ------------------------------------------------------------------ LDS-tiled fp32 kernel (K > 128)
 @pytest.mark.parametrize("m,k,n,kind", [
     (8200, 136, 40, "plain"), (6000, 200, 136, "ln"), (2049, 384, 520, "rms"), (8193, 160, 128, "res"), (3000, 264, 392, "gelu"),
