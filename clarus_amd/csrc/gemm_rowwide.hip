@@ -325,6 +325,7 @@ template <int PRO, int TA, int KS>
 void choose_rw(const GemmP& g, hipStream_t s) {
   RwP p{};
   p.g = g;
+  const int64_t cus = device_cus();
   const int nt = (int)cdiv(g.n, 32);
   const int most = RW_W_MAX / (KS * 1024) & ~1;  // an even count: chunks start on 128-byte lines of the row
   if constexpr (TA == DT_BF16 && KS <= 4) {
@@ -333,7 +334,7 @@ void choose_rw(const GemmP& g, hipStream_t s) {
     // buffer takes LDS, which costs more than it gives at K = 96 (360 x 640, N = 288: 48 -> 61) and where the
     // row groups alone leave CUs idle. The store tiles of four waves have to fit LDS beside W^T (K = 48: N < 456)
     if (nt <= most && rw_lds<KS, true>(nt, (int)g.n) <= RW_LDS_MAX && g.c_dt == DT_BF16 && g.ldc == g.n &&
-        g.n % 64 != 0 && g.n > 64 && !g.has_res && g.act == ACT_NONE && !g.scale && g.out_scale == 1.0f && cdiv(g.m, 128) >= 256) {
+        g.n % 64 != 0 && g.n > 64 && !g.has_res && g.act == ACT_NONE && !g.scale && g.out_scale == 1.0f && cdiv(g.m, 128) >= cus) {
       p.nch = 1;
       p.ntc = nt;
       return launch_rw<PRO, TA, KS, true>(p, s);
@@ -344,7 +345,7 @@ void choose_rw(const GemmP& g, hipStream_t s) {
   auto even = [&](int nch) { return (int)cdiv(nt, 2 * nch) * 2; };
   int nch = (int)cdiv(nt, most);
   if (even(nch + 1) * (nch + 1) < even(nch) * nch) ++nch;
-  while (cdiv(g.m, 128) * nch < 256 && even(nch) > 2) ++nch;
+  while (cdiv(g.m, 128) * nch < cus && even(nch) > 2) ++nch;
   p.ntc = nch == 1 ? nt : even(nch);
   p.nch = (int)cdiv(nt, p.ntc);
   launch_rw<PRO, TA, KS, false>(p, s);

@@ -591,13 +591,14 @@ __global__ void __launch_bounds__(256, 2) dw_tile_kernel(const DwP p, const DwTi
 
 // Lanes per column, columns and slices of dw_tile_kernel for `units` lane units of channels (4 output
 // channels with a gate, else 8), and its tile height, returned. A workgroup takes as long for a tile
-// whatever lanes idle: the cost counts tiles (at least the 512 workgroups that run at once) times a tile's
+// whatever lanes idle: the cost counts tiles (at least the two workgroups per CU that run at once) times a tile's
 // rows. cq is even with a gate (16-byte copies of halves) and at least 16 where the channels reach it:
 // 256 bytes of a pixel or more per slice (us, 720p bf16 without a gate, 9 lanes -> 18: 288 channels
 // 296 -> 250, 144 channels 131 -> 114). Heights: bf16 6 rows, or 2 where 6 leave CUs without a tile
 // (32 x 42, 512 channels, gate: 8.7 -> 6.9 us); fp32, whose 6-row tile fills half a CU's LDS, 2 rows
 // (90 x 160: 1152 channels 35.2 -> 30.0, 2048 with a GELU gate 69.0 -> 51.5).
 static int dw_tile_shape(int64_t units, int64_t n, int64_t H, int64_t W, bool gate, bool f32, DwTileP& g) {
+  const int64_t cus = device_cus();
   double best = 1e300;
   int th = 2;
   const int lo = (int)std::min<int64_t>(gate ? units + (units & 1) : units, 16);
@@ -607,8 +608,8 @@ static int dw_tile_shape(int64_t units, int64_t n, int64_t H, int64_t W, bool ga
     const int64_t nsl = cdiv(units, cq);
     for (int t = 2; t <= (f32 ? 2 : 6); t += 4) {
       const double tiles = (double)nsl * (double)(n * cdiv(H, t) * cdiv(W, tw));
-      if (t == 2 && !f32 && nsl * n * cdiv(H, 6) * cdiv(W, tw) >= 256) continue;
-      const double cost = std::max(tiles / 512.0, 1.0) * (t + 3.0) * (1.0 + 0.5 / tw);
+      if (t == 2 && !f32 && nsl * n * cdiv(H, 6) * cdiv(W, tw) >= cus) continue;
+      const double cost = std::max(tiles / (2.0 * (double)cus), 1.0) * (t + 3.0) * (1.0 + 0.5 / tw);
       if (cost < best * 0.999) {
         best = cost;
         th = t;
