@@ -257,13 +257,13 @@ def test_dwconv_tile_edges(n, h, w, c, gate, hip_bf16):
 
 @pytest.mark.parametrize("n,h,w,c,gate,act", [
     (1, 1, 1, 8, False, None), (1, 3, 2, 16, False, "gelu"),         # smallest slices, images inside one tile
-    (2, 13, 15, 144, False, None), (1, 7, 29, 288, False, None),     # 18 lanes x 14 columns, remainders
+    (2, 13, 15, 144, False, None), (1, 7, 29, 288, False, None),     # remainders
     (1, 26, 33, 1152, False, None), (1, 12, 40, 216, False, "gelu"),  # several slices, the last one partial
     (1, 5, 40, 32, "gelu", None), (2, 9, 17, 528, "gelu", None), (1, 40, 70, 512, True, None)])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 def test_dwconv_tile_forms(n, h, w, c, gate, act, dt, hip_bf16, hip_f32):
-    """dw_tile_kernel without a gate, with fp32 rows and at both tile heights, at the edges of its tiles and
-    channel slices, the bias at an address that is 4-byte aligned only."""
+    """dwconv at the edges of the tiled kernel's tiles and channel slices, in one tile per workgroup, and of the
+    per-pixel kernel for fp32 rows of many channels; the bias at an address that is 4-byte aligned only."""
     from clarus_amd import _lib
     g = gen(c + h)
     x = rnd(g, n, h, w, c, dtype=dt)
@@ -294,14 +294,45 @@ def test_dwconv_routing(h, w, c, gate, dt, tiled, hip_bf16, hip_f32):
     check(got.cpu(), TorchRef(torch.float32, "cpu").dwconv(x, wt, b, gate=gate), f"dwconv routing {h}x{w}x{c} gate={gate} {dt}")
 
 
-def test_dwconv_bf16_in_fp32_out(hip_bf16):
-    """bf16 input with an fp32 output (a combination HipOps does not produce), through the C ABI:
-    640 channels, no gate and with the gate, two images of 37 x 53, against the oracle's fp32
-    result."""
+@pytest.mark.parametrize("n,h,w,c,gate,act,dt,form", [
+    # bf16 without a gate: 6-row tiles, several a workgroup (the next one's copies in flight), remainders both ways
+    (1, 180, 320, 144, False, None, "bf16", "gate=0 th=6 cq=18 tw=14"), (1, 183, 331, 288, False, "gelu", "bf16", "gate=0 th=6 cq=18 tw=14"),
+    (2, 95, 161, 520, False, None, "bf16", "gate=0 th=6"),
+    (1, 181, 322, 256, True, None, "bf16", "gate=1 th=6"), (1, 179, 321, 288, "gelu", None, "bf16", "gate=2 th=6"),
+    # 2-row tiles: bf16 with two buffers, fp32 with one, several a workgroup
+    (1, 60, 64, 576, False, None, "bf16", "gate=0 th=2"), (1, 59, 63, 768, "gelu", None, "bf16", "gate=2 th=2"),
+    (1, 91, 161, 520, False, None, "fp32", "gate=0 th=2"), (1, 90, 165, 400, True, None, "fp32", "gate=1 th=2")])
+def test_dwconv_tile_pipeline(n, h, w, c, gate, act, dt, form, hip_bf16, hip_f32):
+    """dw_tile_kernel past its first tile: both tile heights, with and without a gate, against the oracle."""
+    from clarus_amd import _lib
+    g = gen(c + h)
+    x = rnd(g, n, h, w, c, dtype=torch.float32 if dt == "fp32" else torch.bfloat16)
+    wt, b = rnd(g, c, 1, 3, 3, scale=0.3), rnd(g, c, scale=0.5)
+    got = (hip_f32 if dt == "fp32" else hip_bf16).dwconv(x.cuda(), wt.cuda(), b.cuda(), gate=gate, act=act)
+    assert _lib.last_kernel().startswith(f"dw_tile_kernel {form}"), _lib.last_kernel()
+    check(got.cpu(), TorchRef(torch.float32, "cpu").dwconv(x, wt, b, gate=gate, act=act), f"dwconv pipeline {n}x{h}x{w}x{c} {gate} {dt}")
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("gate,c", [(True, 48), ("gelu", 144), (True, 640)])
+def test_dwconv_dilated_gate(dt, gate, c, hip_bf16, hip_f32):
+    """Dilation 2 with a gate: the per-pixel kernel's gated forms, against the oracle."""
+    from clarus_amd import _lib
+    g = gen(c)
+    x, wt, b = rnd(g, 2, 21, 35, c, dtype=dt), rnd(g, c, 1, 3, 3, scale=0.3), rnd(g, c, scale=0.5)
+    got = (hip_bf16 if dt == torch.bfloat16 else hip_f32).dwconv(x.cuda(), wt.cuda(), b.cuda(), dil=2, gate=gate)
+    assert _lib.last_kernel().startswith(f"dwconv3x3_kernel gate={2 if gate == 'gelu' else 1} dil=2"), _lib.last_kernel()
+    check(got.cpu(), TorchRef(torch.float32, "cpu").dwconv(x, wt, b, dil=2, gate=gate), f"dwconv dil=2 gate={gate} {c} {dt}")
+
+
+@pytest.mark.parametrize("size", [(2, 37, 53, 640), (1, 180, 323, 288)])
+def test_dwconv_bf16_in_fp32_out(size, hip_bf16):
+    """bf16 input with an fp32 output (a combination HipOps does not produce), through the C ABI: no gate
+    and with the gate, a tile or several per workgroup, against the oracle's fp32 result."""
     import ctypes
     from clarus_amd import _lib
     g = gen(12)
-    n, h, w, c = 2, 37, 53, 640
+    n, h, w, c = size
     x, wt, b = rnd(g, n, h, w, c, dtype=torch.bfloat16), rnd(g, c, 1, 3, 3), rnd(g, c)
     taps = wt.float().reshape(c, 9).t().contiguous().cuda()
     for gate in (0, 1):
