@@ -168,10 +168,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc_n(const void* p, uint
 
 // exact-erf GELU (torch.nn.functional.gelu default), x Phi(x) with one branch-free form for every x:
 //   Phi(-a) = exp(-a^2 / 2) N(a) / D(a),  a = |x|,  Phi(a) = 1 - Phi(-a)
-// N, D: a least-squares minimax fit (degrees 3 and 4, own coefficients) of erfcx(a / sqrt 2) / 2, off by
-// at most 4e-9 of max(Phi(-a), 1e-2). All coefficients are positive, so the evaluation loses nothing to
-// cancellation: against 64 bits on N(0, 1) 3.5e-8 (2-norm), with erff 3.8e-8, and no error of
-// 1 + erf(x) for negative x. About 23 VALU slots; erff's two ranges both run in a wave that holds both.
+// N, D: a least-squares minimax fit (degrees 3 and 4, own coefficients) of erfcx(a / sqrt 2) / 2. With the
+// coefficients as fp32 holds them it is off by at most 3.3e-8 of max(Phi(-a), 1e-2), 6.5e-9 of 1, and relative to
+// Phi(-a) itself by 5e-8 up to a = 3, 8e-7 at 4, 1.6e-5 at 6 and 1.2e-4 at 10, where 1 + erf(x) has no digit left
+// below -5.5. All coefficients are positive: against 64 bits on N(0, 1) 3.5e-8 (2-norm), with erff 3.8e-8. About 23
+// VALU slots; erff's two ranges both run in a wave that holds both.
 // a is clamped (past 20 the factor exp is 0) so that N and D stay finite: -inf gives NaN, inf gives inf.
 __device__ __forceinline__ float gelu_erf(float x) {
   const float a = fminf(fabsf(x), 20.f);

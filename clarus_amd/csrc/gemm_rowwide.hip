@@ -11,7 +11,7 @@
 //     lane accumulates 16 consecutive channels of its pixel (two 16-byte stores of bf16). Accumulators start
 //     from the bias.
 //   * W^T sits in LDS in fragment order (one 1 KiB run per tile and 16-k step), the bias, scale and LN-mul
-//     vectors beside it: at most 56 KiB of W^T per workgroup, more channels go to further workgroups of the
+//     vectors beside it: at most 60 KiB of W^T per workgroup, more channels go to further workgroups of the
 //     same XCD, so the rows they share come into one L2 once.
 //   * A lane loads 8 consecutive k of its pixel per step straight into registers, the next tile's rows before
 //     the current tile's products; occupancy hides the rest (bf16 rows: 4 waves per SIMD).
