@@ -98,4 +98,40 @@ __device__ __forceinline__ void fft8(float (&r)[8], float (&i)[8]) {
   }
 }
 
+// ---- a patch on two lanes: half h of the wave holds patch rows 4 h .. 4 h + 3; after the row transforms half 0 takes
+// columns 0 + 4 (both real, as one complex column) and 2, half 1 columns 1 and 3
+
+// v0.upper <-> v1.lower (lanes 32 .. 63 of v0 with lanes 0 .. 31 of v1); its own inverse
+__device__ __forceinline__ void half_swap(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+
+// gain factors of a channel (gp: its 40 complex gains) for half lh: columns 0 + 4 or 1 as W(u) = P z(u) + Q conj z(-u) per
+// component, column 2 or 3 as c. Gains over 64; columns 1 .. 3 doubled; irfft2 keeps the Hermitian part of columns 0
+// and 4, so their gains are symmetrised over u and -u (the two halvings make 1 / 4)
+__device__ __forceinline__ void patch_gains(const f32x2* gp, int lh, float (&pr)[8], float (&pi)[8], float (&qr)[8],
+                                            float (&qi)[8], float (&cr)[8], float (&ci)[8]) {
+  f32x2 a[8], d[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    a[u] = gp[5 * u + lh];
+    d[u] = gp[5 * u + 4];
+    const f32x2 c = gp[5 * u + 2 + lh];
+    cr[u] = c[0] * 0.03125f;  // 2 / 64
+    ci[u] = c[1] * 0.03125f;
+  }
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int m = (8 - u) & 7;
+    const float r0 = a[u][0] + a[m][0], s0 = a[u][1] + a[m][1], r4 = d[u][0] + d[m][0], s4 = d[u][1] + d[m][1];
+    constexpr float q = 0.25f / 64.f;
+    pr[u] = lh ? a[u][0] * 0.03125f : (r0 + s4) * q;
+    pi[u] = lh ? a[u][1] * 0.03125f : (s0 + r4) * q;
+    qr[u] = lh ? 0.f : (r0 - s4) * q;
+    qi[u] = lh ? 0.f : (r4 - s0) * q;
+  }
+}
+
 }  // namespace clarus

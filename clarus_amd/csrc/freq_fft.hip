@@ -32,13 +32,6 @@ namespace {
 constexpr unsigned FP_DROP = 0x7ffffff0u;  // past every range: the access is dropped
 constexpr unsigned FP_RANGE = 0x7fffff00u;
 
-// v0.upper <-> v1.lower (lanes 32 .. 63 of v0 with lanes 0 .. 31 of v1); its own inverse
-__device__ __forceinline__ void fp_swap(float& a, float& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  a = __uint_as_float(r[0]);
-  b = __uint_as_float(r[1]);
-}
-
 // rows 4 h .. 4 h + 3 of a patch -> column spectra: half 0 columns 0 + 4 (a) and 2 (b), half 1 columns 1 and 3
 __device__ __forceinline__ void fp_forward(float (&z)[4][8], float (&ar)[8], float (&ai)[8], float (&br)[8], float (&bi)[8]) {
 #pragma unroll
@@ -51,10 +44,10 @@ __device__ __forceinline__ void fp_forward(float (&z)[4][8], float (&ar)[8], flo
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    fp_swap(ar[j], ar[j + 4]);
-    fp_swap(ai[j], ai[j + 4]);
-    fp_swap(br[j], br[j + 4]);
-    fp_swap(bi[j], bi[j + 4]);
+    half_swap(ar[j], ar[j + 4]);
+    half_swap(ai[j], ai[j + 4]);
+    half_swap(br[j], br[j + 4]);
+    half_swap(bi[j], bi[j + 4]);
   }
   fft8<false>(ar, ai);
   fft8<false>(br, bi);
@@ -66,10 +59,10 @@ __device__ __forceinline__ void fp_inverse(float (&z)[4][8], float (&ar)[8], flo
   fft8<true>(br, bi);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    fp_swap(ar[j], ar[j + 4]);
-    fp_swap(ai[j], ai[j + 4]);
-    fp_swap(br[j], br[j + 4]);
-    fp_swap(bi[j], bi[j + 4]);
+    half_swap(ar[j], ar[j + 4]);
+    half_swap(ai[j], ai[j + 4]);
+    half_swap(br[j], br[j + 4]);
+    half_swap(bi[j], bi[j + 4]);
     z[j][0] = ar[j]; z[j][1] = ar[j + 4];
     z[j][4] = ai[j]; z[j][5] = ai[j + 4];
     z[j][2] = br[j]; z[j][3] = br[j + 4];
@@ -110,28 +103,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) f
   const int d_pt = p.streams * p.span, d_rows = d_pt / pw, d_px = d_pt - d_rows * pw, d_n = d_rows / ph,
             d_py = d_rows - d_n * ph;
   float pr[CORR ? 1 : 8], pi[CORR ? 1 : 8], qr[CORR ? 1 : 8], qi[CORR ? 1 : 8], cr[CORR ? 1 : 8], ci[CORR ? 1 : 8];
-  if constexpr (!CORR) {  // gains over 64, columns 1 .. 3 doubled; columns 0, 4 symmetrised over u and -u
-    const f32x2* gp = reinterpret_cast<const f32x2*>(p.gain) + (int64_t)ch * 40;
-    f32x2 a[8], d[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      a[u] = gp[5 * u + lh];
-      d[u] = gp[5 * u + 4];
-      const f32x2 c = gp[5 * u + 2 + lh];
-      cr[u] = c[0] * 0.03125f;
-      ci[u] = c[1] * 0.03125f;
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int m = (8 - u) & 7;
-      const float r0 = a[u][0] + a[m][0], s0 = a[u][1] + a[m][1], r4 = d[u][0] + d[m][0], s4 = d[u][1] + d[m][1];
-      constexpr float q = 0.25f / 64.f;
-      pr[u] = lh ? a[u][0] * 0.03125f : (r0 + s4) * q;
-      pi[u] = lh ? a[u][1] * 0.03125f : (s0 + r4) * q;
-      qr[u] = lh ? 0.f : (r0 - s4) * q;
-      qi[u] = lh ? 0.f : (r4 - s0) * q;
-    }
-  }
+  if constexpr (!CORR) patch_gains(reinterpret_cast<const f32x2*>(p.gain) + (int64_t)ch * 40, lh, pr, pi, qr, qi, cr, ci);
   const __amdgpu_buffer_rsrc_t xr = buf_rsrc_n(p.x, FP_RANGE), orr = buf_rsrc_n(p.out, FP_RANGE);
   const __amdgpu_buffer_rsrc_t rr = buf_rsrc_n(p.res ? p.res : p.out, FP_RANGE);
   unsigned sh = (unsigned)p.sh, sw = (unsigned)p.sw;

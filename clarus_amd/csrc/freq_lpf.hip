@@ -33,13 +33,6 @@ namespace {
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 constexpr int LF_WAVES = 8;
 
-// v0.upper <-> v1.lower (lanes 32 .. 63 of v0 with lanes 0 .. 31 of v1); its own inverse
-__device__ __forceinline__ void half_swap(float& a, float& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  a = __uint_as_float(r[0]);
-  b = __uint_as_float(r[1]);
-}
-
 template <int KS, bool PRO, int PB>
 __global__ void __launch_bounds__(64 * LF_WAVES, 2) fft_lpf_kernel(const LpfFftP p) {
   constexpr int HL = PRO ? 2 : 1;                 // operand parts: hi (, lo)
@@ -156,29 +149,7 @@ __global__ void __launch_bounds__(64 * LF_WAVES, 2) fft_lpf_kernel(const LpfFftP
       }
       const float bias = p.bias ? p.bias[chl] : 0.f;
       float pr[8], pi[8], qr[8], qi[8], cr[8], ci[8];
-      {
-        const f32x2* g = reinterpret_cast<const f32x2*>(p.gain) + (int64_t)chl * 40;
-        f32x2 a[8], d[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          a[u] = g[5 * u + lh];
-          d[u] = g[5 * u + 4];
-          const f32x2 c = g[5 * u + 2 + lh];
-          cr[u] = c[0] * 0.03125f;  // 2 / 64
-          ci[u] = c[1] * 0.03125f;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int m = (8 - u) & 7;
-          // half 0: g0, g4 symmetrised over u and -u, with 1 / 64 (the two halvings make 1 / 4)
-          const float r0 = a[u][0] + a[m][0], s0 = a[u][1] + a[m][1], r4 = d[u][0] + d[m][0], s4 = d[u][1] + d[m][1];
-          constexpr float q = 0.25f / 64.f;
-          pr[u] = lh ? a[u][0] * 0.03125f : (r0 + s4) * q;
-          pi[u] = lh ? a[u][1] * 0.03125f : (s0 + r4) * q;
-          qr[u] = lh ? 0.f : (r0 - s4) * q;
-          qi[u] = lh ? 0.f : (r4 - s0) * q;
-        }
-      }
+      patch_gains(reinterpret_cast<const f32x2*>(p.gain) + (int64_t)chl * 40, lh, pr, pi, qr, qi, cr, ci);
       for (; i0 < iend; ++i0) {
         const int slot = i0 - ct * PB;
         const int64_t pt = b + slot;

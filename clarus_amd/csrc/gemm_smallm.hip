@@ -234,6 +234,7 @@ void pick_sm(const GemmP& p, bool gate, hipStream_t s) {
 
 }  // namespace
 
+// K = 128 and 256 only: a lane holds half a row, which with fp32 rows of K = 512 is all 256 registers before the operands
 bool gemm_smallm_fits(const GemmP& p, int a_dt, int w_dt) {
   if (w_dt != DT_BF16 || (p.k != 128 && p.k != 256) || p.n % 8 || p.vec_out != 2 || (p.has_res && p.vec_res != 2) ||
       (p.act != ACT_NONE && p.act != ACT_GELU) || p.c_mode != CM_ROWS || cdiv(p.m, 128) * cdiv(p.n, 32) >= ((int64_t)1 << 30))
