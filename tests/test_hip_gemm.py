@@ -1862,3 +1862,76 @@ def test_gemm_f32_per_image(hip_f32):
     got = hip_f32.linear_per_image(qkv.cuda()[..., 288:], w.cuda(), residual=res.cuda())
     assert _lib.last_kernel().startswith("gemm_f32_kernel"), _lib.last_kernel()
     assert_fp32(got.cpu(), TorchRef(torch.float32, "cpu").linear_per_image(qkv[..., 288:], w, residual=res), what="f32 per image")
+
+
+# ------------------------------------------------------------------ strided operands on the row kernels
+STRIDED = [  # tile: 19 all-channel rows, 20 few rows, 21 LDS-tiled fp32, 0 the library's choice
+    (19, "gemm_rowwide", 97, 48, 72, 1, "bf16", dict(lda=24, ldc=16, pro=1)),
+    (19, "gemm_rowwide", 161, 96, 104, 1, "fp32", dict(lda=192, ldc=8, ldr=24, res="fp32", scale=True, pro=3)),
+    (19, "gemm_rowwide", 33000, 48, 72, 1, "bf16", dict(lda=8, ldc=8)),
+    (19, "gemm_rowwide", 129, 40, 64, 1, "bf16", dict(lda=40, ldr=8, res="bf16", act=True)),
+    (0, "gemm_rowwide", 4100, 48, 48, 1, "bf16", dict(lda=96, res="bf16", alias=True)),
+    (0, "gemm_", 700, 48, 144, 1, "bf16", dict(lda=8, skew=4, pro=1)),       # an output at 8-byte addresses
+    (20, "gemm_smallm", 97, 256, 72, 1, "bf16", dict(lda=16, ldc=16, res="fp32", ldr=8, scale=True)),
+    (20, "gemm_smallm", 161, 128, 40, 1, "fp32", dict(lda=8, ldc=24, gate=True, act=True)),
+    (20, "gemm_smallm", 300, 128, 128, 1, "fp32", dict(res="fp32", alias=True)),
+    (21, "gemm_f32", 130, 136, 72, 2, "fp32", dict(lda=20, ldc=8, res="fp32", ldr=4, scale=True)),
+    (21, "gemm_f32", 65, 264, 136, 1, "bf16", dict(lda=4, ldc=8, pro=1, act=True)),
+    (21, "gemm_f32", 200, 160, 64, 1, "fp32", dict(pro=3, res="fp32", alias=True)),
+    (0, "gemm_", 3000, 384, 384, 1, "fp32", dict(skew=1))]                   # an output at 4-byte addresses
+
+
+@pytest.mark.parametrize("tile,kernel,m,k,n,batch,cdt,o", STRIDED)
+def test_row_kernels_strided(tile, kernel, m, k, n, batch, cdt, o, hip_bf16):
+    """Through the C ABI, the row kernels on rows of wider A, C and residual tensors, two batch entries, a residual that
+    is the output, and outputs whose alignment leaves them to the other kernels: against the product in 64 bits (LayerNorm
+    rows of these kernels stay fp32-accurate), columns past N untouched."""
+    import ctypes
+    from clarus_amd import _lib
+    dts = {"bf16": torch.bfloat16, "fp32": torch.float32}
+    g, dt, f32 = gen(tile + m + k), dts[cdt], kernel == "gemm_f32" or k == 384
+    adt = torch.float32 if f32 else torch.bfloat16
+    nw = 2 * n if o.get("gate") else n
+    lda, ldc, ldr = k + o.get("lda", 0), n + o.get("ldc", 0), n + o.get("ldr", 0)
+    xa, wt = rnd(g, batch, m, lda, dtype=adt), rnd(g, batch, nw, k, scale=k ** -0.5, dtype=adt)
+    b, sc = rnd(g, nw), rnd(g, n) if o.get("scale") else None
+    skew = o.get("skew", 0)
+    buf = torch.full((batch * m * ldc + 8,), 7.0, dtype=dt)
+    out = buf[skew:skew + batch * m * ldc].view(batch, m, ldc)
+    res = out if o.get("alias") else rnd(g, batch, m, ldr, dtype=dts[o["res"]]) if "res" in o else None
+    if o.get("alias"):
+        out.copy_(rnd(g, batch, m, ldc, dtype=dt))
+    rows = xa[..., :k].double()
+    if o.get("pro") == 1:
+        rows = rows - rows.mean(-1, keepdim=True)
+    if o.get("pro"):
+        rows = rows / (rows.square().mean(-1, keepdim=True) + 1e-6).sqrt()
+    y = rows @ wt.double().transpose(1, 2) + b.double()
+    y = y[..., :n] * y[..., n:] if o.get("gate") else y
+    y = torch.nn.functional.gelu(y) if o.get("act") else y
+    y = y * (1 if sc is None else sc.double()) * 0.5
+    y = y if res is None else y + res[..., :n].double()
+    dbuf = buf.cuda()
+    cd = dbuf[skew:skew + batch * m * ldc]
+    rd = cd if o.get("alias") else None if res is None else res.cuda()
+    ad, wd, bd, sd = xa.cuda(), wt.cuda(), b.cuda(), None if sc is None else sc.cuda()
+    stats = torch.empty(2 * m, device="cuda")
+    args = _lib.GemmArgs(
+        a=ad.data_ptr(), wt=wd.data_ptr(), c=cd.data_ptr(), bias=bd.data_ptr(), scale=_lib.ptr(sd), res=_lib.ptr(rd),
+        stats=stats.data_ptr(), m=m, n=n, k=k, batch=batch, lda=lda, ldc=ldc, ldr=ldc if o.get("alias") else ldr,
+        a_bstride=m * lda, w_bstride=nw * k, c_bstride=m * ldc, r_bstride=m * (ldc if o.get("alias") else ldr),
+        a_dtype=_lib.dtype_code(adt), w_dtype=_lib.dtype_code(adt), c_dtype=_lib.dtype_code(dt),
+        r_dtype=_lib.dtype_code(res.dtype) if res is not None else 0, pro=o.get("pro", 0), gate=int(bool(o.get("gate"))),
+        act=_lib.ACT_GELU if o.get("act") else 0, ln_eps=1e-6, out_scale=0.5, tile=tile)
+    _lib.check(_lib.load().clarus_hip_gemm(ctypes.byref(args), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "gemm")
+    name = _lib.last_kernel()
+    assert name.startswith(kernel) and not (skew and name.startswith(("gemm_rowwide", "gemm_f32"))), name
+    got = dbuf.cpu()
+    assert (got[:skew] == 7).all() and (got[skew + batch * m * ldc:] == 7).all()
+    got = got[skew:skew + batch * m * ldc].view(batch, m, ldc)
+    assert o.get("alias") or (got[..., n:] == 7).all(), "columns past N written"
+    what = f"strided {name} {m}x{k}x{n}"
+    if dt == torch.bfloat16:
+        assert_bf16(got[..., :n], y.float(), what)
+    else:
+        assert_fp32(got[..., :n], y.float(), rel=1e-5, what=what)
